@@ -29,14 +29,28 @@ namespace pyr {
 constexpr int kTraceBlock = 128;  // rays per workgroup (types.zig:498 trace_block)
 constexpr int kMaxLevels = 21;    // log2_size <= 20
 constexpr uint32_t kMaxSteps = 65536;
+// Scenes from this many instances on test their boxes against a whole wave
+// first. (1920x1080 frames of instance grids: 3 and 6 instances are as fast
+// either way, 16 take 325 us with the test and 330 without, 64 take 476 and
+// 533, 1000 take 802 and 2429.)
+constexpr uint32_t kCullInstances = 8;
 constexpr uint32_t kNotMoved = 4;  // added to the entry axis of a walk that has not left its first cell
 constexpr uint32_t kHit = 32, kMiss = 64;  // values of a finished walk's scale
 
+// Device memory by its address space: a pointer made from a number would be
+// read with flat instructions, which also wait for the LDS; what a traversal
+// kernel only reads at an index that all lanes share goes through the scalar
+// cache.
+#define PYR_GLOBAL __attribute__((address_space(1)))
+#define PYR_CONSTANT __attribute__((address_space(4)))
+typedef const PYR_GLOBAL uint32_t* Words;
+typedef const PYR_GLOBAL uint64_t* Masks;
+
 struct DagView {
-    const uint32_t* nodes;
-    const uint64_t* leaves;
-    const uint32_t* attrs;    // null: default_attribute
-    const uint32_t* palette;  // non-null: attrs holds 4-bit indices into these 16 values
+    Words nodes;
+    Masks leaves;
+    Words attrs;    // null: default_attribute
+    Words palette;  // non-null: attrs holds 4-bit indices into these 16 values
     uint32_t root, log2_size, default_attribute, attr_base;
 };
 
@@ -62,8 +76,7 @@ __device__ __forceinline__ uint32_t brick_bit(uint32_t x, uint32_t y, uint32_t z
 // Node word i, for an index every active lane shares: a scalar load (the
 // node array does not change while a traversal kernel runs).
 __device__ __forceinline__ uint32_t node_uniform(const DagView& g, uint32_t i) {
-    typedef const __attribute__((address_space(4))) uint32_t* ConstWords;
-    return ((ConstWords)g.nodes)[i];
+    return ((const PYR_CONSTANT uint32_t*)g.nodes)[i];
 }
 
 // attributeRank (dag.zig:70-87); stk[s * kTraceBlock] is the node whose
@@ -373,12 +386,31 @@ __device__ __forceinline__ void xform_vector(const float* m, const float v[3], f
 __device__ __forceinline__ bool any_cutout(const PyrScene& s) {
     return (s.cutout_materials[0] | s.cutout_materials[1] | s.cutout_materials[2] | s.cutout_materials[3]) != 0;
 }
-__device__ __forceinline__ bool cutout_here(const PyrInstanceData& in) {
+__device__ __forceinline__ bool cutout_here(const float world_to_object[12]) {
     float w2o = 0.0f;
 #pragma unroll
-    for (int a = 0; a < 3; a++) w2o += in.world_to_object[a] * in.world_to_object[a];
+    for (int a = 0; a < 3; a++) w2o += world_to_object[a] * world_to_object[a];
     return w2o > 0.5f;
 }
+
+// Largest and smallest value of a wave's lanes (all of them active).
+__device__ __forceinline__ float wave_max(float x) {
+    const float u = __uint_as_float(first_lane32(__float_as_uint(x)));
+    if (__ballot(x != u) == 0) return u;
+    auto step = [&](float y) { x = fmaxf(x, y); };
+    auto moved = [&](uint32_t y) { step(__uint_as_float(y)); };
+    moved(dpp32<kDppRowShr1>(__float_as_uint(x), __float_as_uint(x)));
+    moved(dpp32<kDppRowShr2>(__float_as_uint(x), __float_as_uint(x)));
+    moved(dpp32<kDppRowShr4>(__float_as_uint(x), __float_as_uint(x)));
+    moved(dpp32<kDppRowShr8>(__float_as_uint(x), __float_as_uint(x)));
+    moved(dpp32<kDppRowBcast15, 0xa>(__float_as_uint(x), __float_as_uint(x)));
+    moved(dpp32<kDppRowBcast31, 0xc>(__float_as_uint(x), __float_as_uint(x)));
+    return __uint_as_float(lane_read32(__float_as_uint(x), kWave - 1));
+}
+struct Range {
+    float lo, hi;
+};
+__device__ __forceinline__ Range wave_range(float x) { return {-wave_max(-x), wave_max(x)}; }
 
 // SKIPPING: the launch found a material set that may apply (skip flag with
 // transparent materials, or cutout materials); each variant holds one walk,
@@ -388,8 +420,8 @@ template <bool SKIPPING, bool EXT = false>
 __device__ PyrHit trace_scene(const PyrScene& s, const float o[3], const float d[3], float tmin, float tmax,
                               uint32_t ray_mask, uint32_t flags, uint32_t* stk, uint32_t levels,
                               float* p_object = nullptr) {
-    const PyrInstanceData* inst = (const PyrInstanceData*)(uintptr_t)s.instances;
-    const PyrGeometryData* geo = (const PyrGeometryData*)(uintptr_t)s.geometries;
+    const PYR_CONSTANT PyrInstanceData* inst = (const PYR_CONSTANT PyrInstanceData*)(uintptr_t)s.instances;
+    const PYR_CONSTANT PyrGeometryData* geo = (const PYR_CONSTANT PyrGeometryData*)(uintptr_t)s.geometries;
     const float inv[3] = {safe_rcp(d[0]), safe_rcp(d[1]), safe_rcp(d[2])};
     const bool want_attr = (flags & PYR_TRACE_NO_ATTRIBUTE) == 0;
     float best = tmax;
@@ -397,9 +429,9 @@ __device__ PyrHit trace_scene(const PyrScene& s, const float o[3], const float d
     // material sets of the traversal (trace.zig:80, 93-98)
     const uint64_t* skip = SKIPPING && (flags & PYR_TRACE_SKIP_TRANSPARENT) ? s.transparent_materials : nullptr;
     const uint64_t* cut = SKIPPING && any_cutout(s) ? s.cutout_materials : nullptr;
-    for (uint32_t i = 0; i < s.instance_count; i++) {
-        const PyrInstanceData& in = inst[i];
-        if (!(in.flags & PYR_INSTANCE_ACTIVE) || !(in.mask & ray_mask)) continue;
+    auto visit = [&](uint32_t i) {
+        const PYR_CONSTANT PyrInstanceData& in = inst[i];
+        if (!(in.flags & PYR_INSTANCE_ACTIVE) || !(in.mask & ray_mask)) return;
         float lo[3], hi[3];
 #pragma unroll
         for (int a = 0; a < 3; a++) {
@@ -408,35 +440,89 @@ __device__ PyrHit trace_scene(const PyrScene& s, const float o[3], const float d
         }
         const float t0 = fmaxf(fmaxf(fminf(lo[0], hi[0]), fminf(lo[1], hi[1])), fminf(lo[2], hi[2]));
         const float t1 = fminf(fminf(fmaxf(lo[0], hi[0]), fmaxf(lo[1], hi[1])), fmaxf(lo[2], hi[2]));
-        if (!(t0 <= t1)) continue;
-        if (!(fmaxf(t0, tmin) < fminf(t1, best))) continue;
-        const PyrGeometryData& g = geo[in.geometry];
-        if (g.log2_size > levels) continue;  // cannot happen: the stack is sized to the scene's largest edge
+        if (!(t0 <= t1)) return;
+        if (!(fmaxf(t0, tmin) < fminf(t1, best))) return;
+        const PYR_CONSTANT PyrGeometryData& g = geo[in.geometry];
+        if (g.log2_size > levels) return;  // cannot happen: the stack is sized to the scene's largest edge
         DagView v;
-        v.nodes = (const uint32_t*)(uintptr_t)s.nodes + g.node_offset;
-        v.leaves = (const uint64_t*)(uintptr_t)s.leaves + g.leaf_offset;
-        v.attrs = (g.flags & PYR_GEOMETRY_HAS_ATTRIBUTES) ? (const uint32_t*)(uintptr_t)s.attributes + g.attribute_offset
+        v.nodes = (Words)(uintptr_t)s.nodes + g.node_offset;
+        v.leaves = (Masks)(uintptr_t)s.leaves + g.leaf_offset;
+        v.attrs = (g.flags & PYR_GEOMETRY_HAS_ATTRIBUTES) ? (Words)(uintptr_t)s.attributes + g.attribute_offset
                                                          : nullptr;
-        v.palette = (g.flags & PYR_GEOMETRY_PALETTE) ? (const uint32_t*)(uintptr_t)s.attributes + g.palette_offset
+        v.palette = (g.flags & PYR_GEOMETRY_PALETTE) ? (Words)(uintptr_t)s.attributes + g.palette_offset
                                                      : nullptr;
         v.root = g.root;
         v.log2_size = g.log2_size;
         v.default_attribute = g.default_attribute;
         v.attr_base = 0;
-        float oo[3], dv[3];
-        xform_point(in.world_to_object, o, oo);
-        xform_vector(in.world_to_object, d, dv);
+        float m[12], oo[3], dv[3];
+#pragma unroll
+        for (int k = 0; k < 12; k++) m[k] = in.world_to_object[k];
+        xform_point(m, o, oo);
+        xform_vector(m, d, dv);
         DagHitD h;
         // with both sets null the skipping walk returns what the plain one does
-        const uint64_t* icut = cut && cutout_here(in) ? cut : nullptr;
+        const uint64_t* icut = cut && cutout_here(m) ? cut : nullptr;
         if (walk<SKIPPING>(v, oo, dv, tmin, best, want_attr, stk, &h, skip, icut)) {
             best = h.t;
             result = to_hit(true, h, i);
             if (EXT)
 #pragma unroll
                 for (int a = 0; a < 3; a++) p_object[a] = oo[a] + dv[a] * h.t;
-            if (flags & PYR_TRACE_ANY_HIT) return result;
+            // (an any-hit ray is over: no box begins before minus infinity)
+            if (flags & PYR_TRACE_ANY_HIT) best = -__builtin_inff();
         }
+    };
+    if (s.instance_count < kCullInstances) {
+        for (uint32_t i = 0; i < s.instance_count; i++) visit(i);
+        return result;
+    }
+    // The test of every box by every ray was most of a frame of many instances
+    // (1000 instances, 1920x1080: 3.59 ms, 2.43 with the tables read through
+    // the scalar cache, 0.80 with the test below; 64 instances 0.60, 0.53,
+    // 0.48 ms). So each lane tests another instance's box against all rays of the wave at
+    // once: the boxes' slab distances over the range of the wave's origins and
+    // reciprocal directions. Subtraction and multiplication round monotonically,
+    // so the range of the corners' products holds every ray's own product, and
+    // an instance that fails the test fails it for each of the rays. Those that
+    // pass are visited in their order. (Undefined and infinite numbers give no
+    // range: then every instance is a candidate.)
+    Range ro[3], ri[3];
+    bool finite = true;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        finite &= fabsf(o[a]) < __builtin_inff() && fabsf(inv[a]) < __builtin_inff() && inv[a] != 0.0f;
+        ro[a] = wave_range(o[a]);
+        ri[a] = wave_range(inv[a]);
+    }
+    const bool ranges = __ballot(!finite) == 0;
+    const float near = -wave_max(-tmin);
+    for (uint32_t base = 0; base < s.instance_count; base += kWave) {
+        const uint32_t j = base + lane_id();
+        const float far = wave_max(best);
+        bool candidate = j < s.instance_count;
+        if (candidate) {
+            const PYR_CONSTANT PyrInstanceData& in = inst[j];
+            candidate = (in.flags & PYR_INSTANCE_ACTIVE) && (in.mask & ray_mask);
+            if (ranges) {
+                float t0 = near, t1 = far;
+#pragma unroll
+                for (int a = 0; a < 3; a++) {
+                    const float b[4] = {in.bounds_min[a] - ro[a].lo, in.bounds_min[a] - ro[a].hi,
+                                        in.bounds_max[a] - ro[a].lo, in.bounds_max[a] - ro[a].hi};
+                    float lo = __builtin_inff(), hi = -__builtin_inff();
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        lo = fminf(lo, fminf(b[k] * ri[a].lo, b[k] * ri[a].hi));
+                        hi = fmaxf(hi, fmaxf(b[k] * ri[a].lo, b[k] * ri[a].hi));
+                    }
+                    t0 = fmaxf(t0, lo);
+                    t1 = fminf(t1, hi);
+                }
+                candidate = candidate && t0 <= t1;
+            }
+        }
+        for (uint64_t m = __ballot(candidate); m; m &= m - 1) visit(base + (uint32_t)__builtin_ctzll(m));
     }
     return result;
 }
@@ -447,15 +533,18 @@ extern __shared__ uint32_t s_stk[];
 
 __host__ __device__ constexpr uint32_t stack_bytes(uint32_t levels) { return levels * kTraceBlock * 4u; }
 
+// Scene kernels keep every lane of a wave active (the instance test works on
+// all of them): lanes past the last ray repeat it.
+
 template <bool SKIPPING>
 __global__ void __launch_bounds__(kTraceBlock) k_trace_scene(const PyrScene* scene, const PyrRay* rays, PyrHit* hits,
                                                               uint32_t count, uint32_t ray_mask, uint32_t flags,
                                                               uint32_t levels) {
-    const uint32_t i = blockIdx.x * kTraceBlock + threadIdx.x;
-    if (i >= count) return;
-    const PyrRay r = rays[i];
-    hits[i] = trace_scene<SKIPPING>(*scene, r.origin, r.direction, r.tmin, r.tmax, ray_mask, flags, s_stk + threadIdx.x,
-                                    levels);
+    const uint32_t i = blockIdx.x * kTraceBlock + threadIdx.x, k = min(i, count - 1);
+    const PyrRay r = rays[k];
+    const PyrHit h = trace_scene<SKIPPING>(*scene, r.origin, r.direction, r.tmin, r.tmax, ray_mask, flags,
+                                           s_stk + threadIdx.x, levels);
+    if (i < count) hits[i] = h;
 }
 
 // extendedHit and hitNormal (trace.zig:125-157): the voxel from the object
@@ -497,13 +586,12 @@ template <bool SKIPPING>
 __global__ void __launch_bounds__(kTraceBlock) k_trace_scene_ex(const PyrScene* scene, const PyrRay* rays,
                                                                  PyrHitEx* hits, uint32_t count, uint32_t ray_mask,
                                                                  uint32_t flags, uint32_t levels) {
-    const uint32_t i = blockIdx.x * kTraceBlock + threadIdx.x;
-    if (i >= count) return;
-    const PyrRay r = rays[i];
+    const uint32_t i = blockIdx.x * kTraceBlock + threadIdx.x, k = min(i, count - 1);
+    const PyrRay r = rays[k];
     float po[3] = {0.0f, 0.0f, 0.0f};
     const PyrHit h = trace_scene<SKIPPING, true>(*scene, r.origin, r.direction, r.tmin, r.tmax, ray_mask, flags,
                                                   s_stk + threadIdx.x, levels, po);
-    store_extended(*scene, r.origin, r.direction, h, po, hits + i);
+    if (i < count) store_extended(*scene, r.origin, r.direction, h, po, hits + i);
 }
 
 __global__ void __launch_bounds__(kTraceBlock) k_trace_dag(DagView g, const PyrRay* rays, PyrHit* hits,
@@ -565,11 +653,12 @@ template <bool SKIPPING>
 __global__ void __launch_bounds__(kTraceBlock) k_render_scene(const PyrScene* scene, PyrCamera cam, const float* w2v,
                                                                PyrHit* hits, float* depth, uint32_t ray_mask,
                                                                uint32_t flags, uint32_t levels) {
-    const uint32_t x = blockIdx.x * 16 + (threadIdx.x & 15), y = blockIdx.y * 8 + (threadIdx.x >> 4);
-    if (x >= cam.width || y >= cam.height) return;
+    const uint32_t px = blockIdx.x * 16 + (threadIdx.x & 15), py = blockIdx.y * 8 + (threadIdx.x >> 4);
+    const uint32_t x = min(px, cam.width - 1), y = min(py, cam.height - 1);
     float o[3], d[3], tmin, tmax;
     camera_ray(cam, x, y, o, d, &tmin, &tmax);
     PyrHit h = trace_scene<SKIPPING>(*scene, o, d, tmin, tmax, ray_mask, flags, s_stk + threadIdx.x, levels);
+    if (px >= cam.width || py >= cam.height) return;
     const uint64_t i = (uint64_t)y * cam.width + x;
     if (hits) hits[i] = h;
     if (depth) {
@@ -613,10 +702,10 @@ __global__ void __launch_bounds__(kTraceBlock) k_trace_shadow(DagView g, const P
 
 DagView view_of(const PyrhipDag& d) {
     DagView g;
-    g.nodes = (const uint32_t*)(uintptr_t)d.nodes;
-    g.leaves = (const uint64_t*)(uintptr_t)d.leaves;
-    g.attrs = (const uint32_t*)(uintptr_t)d.attrs;
-    g.palette = d.attrs ? (const uint32_t*)(uintptr_t)d.palette : nullptr;
+    g.nodes = (Words)(uintptr_t)d.nodes;
+    g.leaves = (Masks)(uintptr_t)d.leaves;
+    g.attrs = (Words)(uintptr_t)d.attrs;
+    g.palette = d.attrs ? (Words)(uintptr_t)d.palette : nullptr;
     g.root = d.root;
     g.log2_size = d.log2_size;
     g.default_attribute = d.default_attribute;
