@@ -24,9 +24,9 @@ thread_local char g_diag[512];
 // to these rays (the skip flag with transparent materials, or cutout
 // materials), which selects the walk that checks them
 PyrResult launch_trace_scene(const PyrScene* scene_dev, uint64_t rays, uint64_t hits, uint32_t count,
-                             uint32_t ray_mask, uint32_t flags, uint32_t levels, bool skipping, hipStream_t s);
+                             uint32_t ray_mask, uint32_t flags, uint32_t levels, uint32_t instances, bool skipping, hipStream_t s);
 PyrResult launch_render_scene(const PyrScene* scene_dev, const PyrCamera& cam, const float* w2v_dev, uint64_t hits,
-                              uint64_t depth, uint32_t ray_mask, uint32_t flags, uint32_t levels, bool skipping,
+                              uint64_t depth, uint32_t ray_mask, uint32_t flags, uint32_t levels, uint32_t instances, bool skipping,
                               hipStream_t s);
 
 namespace {
@@ -159,6 +159,7 @@ struct PyrContext {
     float* w2v_dev = nullptr;
     uint32_t history = 0;
     uint32_t views = 0;
+    uint32_t scene_instances = 0;  // of the committed scene
     uint32_t scene_levels = 3;  // largest geometry edge (log2) referenced by the committed instances
     // material table (context.zig:1948-1964): host copy for the transparent /
     // cutout sets of the next commit, device copy for the caller's kernels
@@ -1121,6 +1122,7 @@ PYR_API PyrResult pyr_commit(PyrContext* ctx, const PyrFrameInfo* info) {
     // host staging above is stack memory: finish the copies before returning
     if (r == PYR_OK) r = hip_check(hipStreamSynchronize(s), "commit");
     // a failed commit may have replaced some tables: keep a stack that fits both scenes
+    ctx->scene_instances = (uint32_t)ins.size();  // (only a launch shape depends on it)
     ctx->scene_levels = r == PYR_OK ? levels : std::max(ctx->scene_levels, levels);
     const bool tr = (sc.transparent_materials[0] | sc.transparent_materials[1] | sc.transparent_materials[2] |
                      sc.transparent_materials[3]) != 0;
@@ -1147,7 +1149,7 @@ PYR_API PyrResult pyr_trace(PyrContext* ctx, uint64_t rays, uint64_t hits, uint3
     if (!ctx || (count && (!rays || !hits))) return fail(PYR_ERROR_INVALID_ARGUMENT, "null argument");
     const bool skipping = ((flags & PYR_TRACE_SKIP_TRANSPARENT) && ctx->scene_transparent) || ctx->scene_cutout;
     PyrResult r = launch_trace_scene(ctx->scene_dev, rays, hits, count, ray_mask ? ray_mask : 0xFFFFFFFFu, flags,
-                                     ctx->scene_levels, skipping, ctx->stream);
+                                     ctx->scene_levels, ctx->scene_instances, skipping, ctx->stream);
     if (r == PYR_OK && (ctx->flags & PYR_CREATE_DEBUG)) r = hip_check(hipStreamSynchronize(ctx->stream), "trace");
     return r;
 }
@@ -1251,7 +1253,7 @@ PYR_API PyrResult pyr_render(PyrContext* ctx, PyrView view, const PyrCamera* cam
     if (r == PYR_OK)
         r = launch_render_scene(ctx->scene_dev, *camera, ctx->w2v_dev, t->hits, t->depth,
                                 t->ray_mask ? t->ray_mask : 0xFFFFFFFFu, t->flags & PYR_TRACE_NO_ATTRIBUTE,
-                                ctx->scene_levels, ctx->scene_cutout, ctx->stream);
+                                ctx->scene_levels, ctx->scene_instances, ctx->scene_cutout, ctx->stream);
     // w2v is host stack memory
     if (r == PYR_OK) r = hip_check(hipStreamSynchronize(ctx->stream), "render");
     return r;

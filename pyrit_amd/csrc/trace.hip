@@ -34,6 +34,14 @@ constexpr uint32_t kMaxSteps = 65536;
 // either way, 16 take 325 us with the test and 330 without, 64 take 476 and
 // 533, 1000 take 802 and 2429.)
 constexpr uint32_t kCullInstances = 8;
+// A launch whose rays make fewer waves than this takes fewer rays per wave: a
+// chip with idle slots gains from waves that diverge less and whose boxes
+// are smaller, a full one loses by the repeated lanes. The chip holds 8192
+// waves. One DAG (or a few instances): 1000 diffuse rays 55 -> 36 us, 16000
+// 88 -> 73, 64000 84 -> 81; 8192 waves take 89 us for the 64000, 16384 take
+// 115. Instances: a 640x360 frame of 64 takes 468 us with full waves, 383 with
+// at least 8192, 340 with 16384, 354 with 32768; of 1000: 633, 500, 432, 557.
+constexpr uint32_t kRayWaves = 4096, kSceneWaves = 16384;
 constexpr uint32_t kNotMoved = 4;  // added to the entry axis of a walk that has not left its first cell
 constexpr uint32_t kHit = 32, kMiss = 64;  // values of a finished walk's scale
 
@@ -533,18 +541,30 @@ extern __shared__ uint32_t s_stk[];
 
 __host__ __device__ constexpr uint32_t stack_bytes(uint32_t levels) { return levels * kTraceBlock * 4u; }
 
-// Scene kernels keep every lane of a wave active (the instance test works on
-// all of them): lanes past the last ray repeat it.
+// A wave holds per_wave rays (a power of two); its other lanes repeat
+// them, so every lane of a wave stays active (the instance test works on all).
+__device__ __forceinline__ uint32_t shared_ray(uint32_t per_wave) {
+    const uint32_t wave = blockIdx.x * (kTraceBlock / kWave) + threadIdx.x / kWave;
+    return wave * per_wave + (lane_id() & (per_wave - 1));
+}
+// pixels of a frame: a wave holds a tile of 2^tile_x by 2^tile_y pixels, and
+// the two waves of a workgroup lie one above the other
+__device__ __forceinline__ void shared_pixel(uint32_t tile, uint32_t* x, uint32_t* y) {
+    const uint32_t tx = tile & 0xFFu, ty = tile >> 8, i = lane_id() & ((1u << (tx + ty)) - 1);
+    *x = (blockIdx.x << tx) + (i & ((1u << tx) - 1));
+    *y = ((blockIdx.y * (kTraceBlock / kWave) + threadIdx.x / kWave) << ty) + (i >> tx);
+}
+__device__ __forceinline__ bool own_lane(uint32_t per_wave) { return lane_id() < per_wave; }
 
 template <bool SKIPPING>
 __global__ void __launch_bounds__(kTraceBlock) k_trace_scene(const PyrScene* scene, const PyrRay* rays, PyrHit* hits,
                                                               uint32_t count, uint32_t ray_mask, uint32_t flags,
-                                                              uint32_t levels) {
-    const uint32_t i = blockIdx.x * kTraceBlock + threadIdx.x, k = min(i, count - 1);
+                                                              uint32_t levels, uint32_t per_wave) {
+    const uint32_t i = shared_ray(per_wave), k = min(i, count - 1);
     const PyrRay r = rays[k];
     const PyrHit h = trace_scene<SKIPPING>(*scene, r.origin, r.direction, r.tmin, r.tmax, ray_mask, flags,
                                            s_stk + threadIdx.x, levels);
-    if (i < count) hits[i] = h;
+    if (i < count && own_lane(per_wave)) hits[i] = h;
 }
 
 // extendedHit and hitNormal (trace.zig:125-157): the voxel from the object
@@ -585,24 +605,24 @@ __device__ __forceinline__ void store_extended(const PyrScene& s, const float o[
 template <bool SKIPPING>
 __global__ void __launch_bounds__(kTraceBlock) k_trace_scene_ex(const PyrScene* scene, const PyrRay* rays,
                                                                  PyrHitEx* hits, uint32_t count, uint32_t ray_mask,
-                                                                 uint32_t flags, uint32_t levels) {
-    const uint32_t i = blockIdx.x * kTraceBlock + threadIdx.x, k = min(i, count - 1);
+                                                                 uint32_t flags, uint32_t levels, uint32_t per_wave) {
+    const uint32_t i = shared_ray(per_wave), k = min(i, count - 1);
     const PyrRay r = rays[k];
     float po[3] = {0.0f, 0.0f, 0.0f};
     const PyrHit h = trace_scene<SKIPPING, true>(*scene, r.origin, r.direction, r.tmin, r.tmax, ray_mask, flags,
                                                   s_stk + threadIdx.x, levels, po);
-    if (i < count) store_extended(*scene, r.origin, r.direction, h, po, hits + i);
+    if (i < count && own_lane(per_wave)) store_extended(*scene, r.origin, r.direction, h, po, hits + i);
 }
 
 __global__ void __launch_bounds__(kTraceBlock) k_trace_dag(DagView g, const PyrRay* rays, PyrHit* hits,
-                                                            uint32_t count, uint32_t flags) {
-    const uint32_t i = blockIdx.x * kTraceBlock + threadIdx.x;
+                                                            uint32_t count, uint32_t flags, uint32_t per_wave) {
+    const uint32_t i = shared_ray(per_wave);
     if (i >= count) return;
     const PyrRay r = rays[i];
     DagHitD h;
     bool f = walk<false>(g, r.origin, r.direction, r.tmin, r.tmax, (flags & PYR_TRACE_NO_ATTRIBUTE) == 0,
                   s_stk + threadIdx.x, &h);
-    hits[i] = to_hit(f, h, 0);
+    if (own_lane(per_wave)) hits[i] = to_hit(f, h, 0);
 }
 
 // cameraRay (render.zig:16-32) for pixel centre + jitter (render.zig:133-141)
@@ -631,14 +651,15 @@ __device__ __forceinline__ void camera_ray(const PyrCamera& c, uint32_t x, uint3
 
 // 8x16 pixel tiles per workgroup keep a wave's rays coherent
 __global__ void __launch_bounds__(kTraceBlock) k_trace_camera(DagView g, PyrCamera cam, PyrHit* hits,
-                                                               uint32_t flags) {
-    const uint32_t x = blockIdx.x * 16 + (threadIdx.x & 15), y = blockIdx.y * 8 + (threadIdx.x >> 4);
+                                                               uint32_t flags, uint32_t tile) {
+    uint32_t x, y;
+    shared_pixel(tile, &x, &y);
     if (x >= cam.width || y >= cam.height) return;
     float o[3], d[3], tmin, tmax;
     camera_ray(cam, x, y, o, d, &tmin, &tmax);
     DagHitD h;
     bool f = walk<false>(g, o, d, tmin, tmax, (flags & PYR_TRACE_NO_ATTRIBUTE) == 0, s_stk + threadIdx.x, &h);
-    hits[(uint64_t)y * cam.width + x] = to_hit(f, h, 0);
+    if (own_lane(1u << ((tile & 0xFFu) + (tile >> 8)))) hits[(uint64_t)y * cam.width + x] = to_hit(f, h, 0);
 }
 
 __global__ void __launch_bounds__(kTraceBlock) k_camera_rays(PyrCamera cam, PyrRay* rays) {
@@ -652,13 +673,14 @@ __global__ void __launch_bounds__(kTraceBlock) k_camera_rays(PyrCamera cam, PyrR
 template <bool SKIPPING>
 __global__ void __launch_bounds__(kTraceBlock) k_render_scene(const PyrScene* scene, PyrCamera cam, const float* w2v,
                                                                PyrHit* hits, float* depth, uint32_t ray_mask,
-                                                               uint32_t flags, uint32_t levels) {
-    const uint32_t px = blockIdx.x * 16 + (threadIdx.x & 15), py = blockIdx.y * 8 + (threadIdx.x >> 4);
+                                                               uint32_t flags, uint32_t levels, uint32_t tile) {
+    uint32_t px, py;
+    shared_pixel(tile, &px, &py);
     const uint32_t x = min(px, cam.width - 1), y = min(py, cam.height - 1);
     float o[3], d[3], tmin, tmax;
     camera_ray(cam, x, y, o, d, &tmin, &tmax);
     PyrHit h = trace_scene<SKIPPING>(*scene, o, d, tmin, tmax, ray_mask, flags, s_stk + threadIdx.x, levels);
-    if (px >= cam.width || py >= cam.height) return;
+    if (px >= cam.width || py >= cam.height || !own_lane(1u << ((tile & 0xFFu) + (tile >> 8)))) return;
     const uint64_t i = (uint64_t)y * cam.width + x;
     if (hits) hits[i] = h;
     if (depth) {
@@ -678,12 +700,12 @@ __global__ void __launch_bounds__(kTraceBlock) k_render_scene(const PyrScene* sc
 // moved 1e-3 voxel along the face normal toward the sun, any hit
 __global__ void __launch_bounds__(kTraceBlock) k_trace_shadow(DagView g, const PyrRay* rays, const PyrHit* prim,
                                                                float sx, float sy, float sz, uint32_t* out,
-                                                               uint32_t count) {
-    const uint32_t i = blockIdx.x * kTraceBlock + threadIdx.x;
+                                                               uint32_t count, uint32_t per_wave) {
+    const uint32_t i = shared_ray(per_wave);
     if (i >= count) return;
     const PyrHit h = prim[i];
     if (h.instance == PYR_NO_HIT) {
-        out[i] = 0xFFFFFFFFu;
+        if (own_lane(per_wave)) out[i] = 0xFFFFFFFFu;
         return;
     }
     const PyrRay r = rays[i];
@@ -697,7 +719,31 @@ __global__ void __launch_bounds__(kTraceBlock) k_trace_shadow(DagView g, const P
         o[a] = r.origin[a] + r.direction[a] * h.t + nrm * 1e-3f;
     }
     DagHitD sh;
-    out[i] = walk<false>(g, o, d, 0.0f, PYR_FLT_MAX, false, s_stk + threadIdx.x, &sh) ? 1u : 0u;
+    const uint32_t dark = walk<false>(g, o, d, 0.0f, PYR_FLT_MAX, false, s_stk + threadIdx.x, &sh) ? 1u : 0u;
+    if (own_lane(per_wave)) out[i] = dark;
+}
+
+// Rays of a wave: 64, or fewer while `count` rays make fewer than `waves`
+// waves.
+uint32_t rays_per_wave(uint64_t count, uint32_t waves) {
+    uint32_t p = kWave;
+    while (p > 1 && count * 2 <= (uint64_t)waves * p) p /= 2;
+    return p;
+}
+dim3 ray_grid(uint32_t count, uint32_t per_wave) {
+    const uint32_t per_block = per_wave * (kTraceBlock / kWave);
+    return dim3((uint32_t)(((uint64_t)count + per_block - 1) / per_block));
+}
+// tile of a frame's waves: 16 x 4 pixels, halved in turn down to one
+uint32_t frame_tile(uint32_t width, uint32_t height, uint32_t waves) {
+    const uint32_t p = rays_per_wave((uint64_t)width * height, waves);
+    const uint32_t bits = (uint32_t)__builtin_ctz(p);
+    const uint32_t ty = bits / 2 < 2 ? bits / 2 : 2;
+    return (bits - ty) | (ty << 8);
+}
+dim3 frame_grid(uint32_t width, uint32_t height, uint32_t tile) {
+    const uint32_t w = 1u << (tile & 0xFFu), h = (kTraceBlock / kWave) << (tile >> 8);
+    return dim3((width + w - 1) / w, (height + h - 1) / h);
 }
 
 DagView view_of(const PyrhipDag& d) {
@@ -714,40 +760,44 @@ DagView view_of(const PyrhipDag& d) {
 }
 
 PyrResult launch_trace_scene(const PyrScene* scene_dev, uint64_t rays, uint64_t hits, uint32_t count,
-                             uint32_t ray_mask, uint32_t flags, uint32_t levels, bool skipping, hipStream_t s) {
+                             uint32_t ray_mask, uint32_t flags, uint32_t levels, uint32_t instances, bool skipping,
+                             hipStream_t s) {
     if (count == 0) return PYR_OK;
     if (levels < 3 || levels > kMaxLevels) return fail(PYR_ERROR_INVALID_ARGUMENT, "scene levels %u", levels);
-    const dim3 grid((count + kTraceBlock - 1) / kTraceBlock);
+    const uint32_t per_wave = rays_per_wave(count, instances < kCullInstances ? kRayWaves : kSceneWaves);
+    const dim3 grid = ray_grid(count, per_wave);
     if (flags & PYR_TRACE_EXTENDED) {
         if (skipping)
             hipLaunchKernelGGL(k_trace_scene_ex<true>, grid, dim3(kTraceBlock), stack_bytes(levels), s, scene_dev,
                                (const PyrRay*)(uintptr_t)rays, (PyrHitEx*)(uintptr_t)hits, count, ray_mask, flags,
-                               levels);
+                               levels, per_wave);
         else
             hipLaunchKernelGGL(k_trace_scene_ex<false>, grid, dim3(kTraceBlock), stack_bytes(levels), s, scene_dev,
                                (const PyrRay*)(uintptr_t)rays, (PyrHitEx*)(uintptr_t)hits, count, ray_mask, flags,
-                               levels);
+                               levels, per_wave);
     } else if (skipping)
         hipLaunchKernelGGL(k_trace_scene<true>, grid, dim3(kTraceBlock), stack_bytes(levels), s, scene_dev,
-                           (const PyrRay*)(uintptr_t)rays, (PyrHit*)(uintptr_t)hits, count, ray_mask, flags, levels);
+                           (const PyrRay*)(uintptr_t)rays, (PyrHit*)(uintptr_t)hits, count, ray_mask, flags, levels, per_wave);
     else
         hipLaunchKernelGGL(k_trace_scene<false>, grid, dim3(kTraceBlock), stack_bytes(levels), s, scene_dev,
-                           (const PyrRay*)(uintptr_t)rays, (PyrHit*)(uintptr_t)hits, count, ray_mask, flags, levels);
+                           (const PyrRay*)(uintptr_t)rays, (PyrHit*)(uintptr_t)hits, count, ray_mask, flags, levels, per_wave);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? PYR_OK : fail(PYR_ERROR_CUDA, "trace launch: %s", hipGetErrorString(e));
 }
 
 PyrResult launch_render_scene(const PyrScene* scene_dev, const PyrCamera& cam, const float* w2v_dev, uint64_t hits,
-                              uint64_t depth, uint32_t ray_mask, uint32_t flags, uint32_t levels, bool skipping,
+                              uint64_t depth, uint32_t ray_mask, uint32_t flags, uint32_t levels, uint32_t instances,
+                              bool skipping,
                               hipStream_t s) {
     if (levels < 3 || levels > kMaxLevels) return fail(PYR_ERROR_INVALID_ARGUMENT, "scene levels %u", levels);
-    dim3 grid((cam.width + 15) / 16, (cam.height + 7) / 8);
+    const uint32_t tile = frame_tile(cam.width, cam.height, instances < kCullInstances ? kRayWaves : kSceneWaves);
+    const dim3 grid = frame_grid(cam.width, cam.height, tile);
     if (skipping)
         hipLaunchKernelGGL(k_render_scene<true>, grid, dim3(kTraceBlock), stack_bytes(levels), s, scene_dev, cam,
-                           w2v_dev, (PyrHit*)(uintptr_t)hits, (float*)(uintptr_t)depth, ray_mask, flags, levels);
+                           w2v_dev, (PyrHit*)(uintptr_t)hits, (float*)(uintptr_t)depth, ray_mask, flags, levels, tile);
     else
         hipLaunchKernelGGL(k_render_scene<false>, grid, dim3(kTraceBlock), stack_bytes(levels), s, scene_dev, cam,
-                           w2v_dev, (PyrHit*)(uintptr_t)hits, (float*)(uintptr_t)depth, ray_mask, flags, levels);
+                           w2v_dev, (PyrHit*)(uintptr_t)hits, (float*)(uintptr_t)depth, ray_mask, flags, levels, tile);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? PYR_OK : fail(PYR_ERROR_CUDA, "render launch: %s", hipGetErrorString(e));
 }
@@ -764,9 +814,10 @@ PYR_API PyrResult pyrhip_trace_dag(const PyrhipDag* dag, uint64_t rays, uint64_t
     if (!dag || (count && (!rays || !hits))) return fail(PYR_ERROR_INVALID_ARGUMENT, "null argument");
     if (dag->log2_size < 3 || dag->log2_size > 20) return fail(PYR_ERROR_INVALID_ARGUMENT, "log2_size");
     if (count == 0) return PYR_OK;
-    hipLaunchKernelGGL(k_trace_dag, dim3((count + kTraceBlock - 1) / kTraceBlock), dim3(kTraceBlock),
+    const uint32_t per_wave = rays_per_wave(count, kRayWaves);
+    hipLaunchKernelGGL(k_trace_dag, ray_grid(count, per_wave), dim3(kTraceBlock),
                        stack_bytes(dag->log2_size), (hipStream_t)stream, view_of(*dag), (const PyrRay*)(uintptr_t)rays, (PyrHit*)(uintptr_t)hits,
-                       count, flags);
+                       count, flags, per_wave);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? PYR_OK : fail(PYR_ERROR_CUDA, "trace launch: %s", hipGetErrorString(e));
 }
@@ -777,10 +828,10 @@ PYR_API PyrResult pyrhip_trace_camera(const PyrhipDag* dag, const PyrCamera* cam
     if (!dag || !camera || !hits) return fail(PYR_ERROR_INVALID_ARGUMENT, "null argument");
     if (dag->log2_size < 3 || dag->log2_size > 20) return fail(PYR_ERROR_INVALID_ARGUMENT, "log2_size");
     if (camera->width == 0 || camera->height == 0) return PYR_OK;
-    dim3 grid((camera->width + 15) / 16, (camera->height + 7) / 8);
-    hipLaunchKernelGGL(k_trace_camera, grid, dim3(kTraceBlock), stack_bytes(dag->log2_size), (hipStream_t)stream,
+    const uint32_t tile = frame_tile(camera->width, camera->height, kRayWaves);
+    hipLaunchKernelGGL(k_trace_camera, frame_grid(camera->width, camera->height, tile), dim3(kTraceBlock), stack_bytes(dag->log2_size), (hipStream_t)stream,
                        view_of(*dag), *camera,
-                       (PyrHit*)(uintptr_t)hits, flags);
+                       (PyrHit*)(uintptr_t)hits, flags, tile);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? PYR_OK : fail(PYR_ERROR_CUDA, "trace launch: %s", hipGetErrorString(e));
 }
@@ -802,9 +853,11 @@ PYR_API PyrResult pyrhip_trace_shadow(const PyrhipDag* dag, uint64_t rays, uint6
     if (!dag || !sun || (count && (!rays || !hits || !out))) return fail(PYR_ERROR_INVALID_ARGUMENT, "null argument");
     if (dag->log2_size < 3 || dag->log2_size > 20) return fail(PYR_ERROR_INVALID_ARGUMENT, "log2_size");
     if (count == 0) return PYR_OK;
-    hipLaunchKernelGGL(k_trace_shadow, dim3((count + kTraceBlock - 1) / kTraceBlock), dim3(kTraceBlock),
+    const uint32_t per_wave = rays_per_wave(count, kRayWaves);
+    hipLaunchKernelGGL(k_trace_shadow, ray_grid(count, per_wave), dim3(kTraceBlock),
                        stack_bytes(dag->log2_size), (hipStream_t)stream, view_of(*dag), (const PyrRay*)(uintptr_t)rays,
-                       (const PyrHit*)(uintptr_t)hits, sun[0], sun[1], sun[2], (uint32_t*)(uintptr_t)out, count);
+                       (const PyrHit*)(uintptr_t)hits, sun[0], sun[1], sun[2], (uint32_t*)(uintptr_t)out, count,
+                       per_wave);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? PYR_OK : fail(PYR_ERROR_CUDA, "trace launch: %s", hipGetErrorString(e));
 }
