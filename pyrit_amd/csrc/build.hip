@@ -41,6 +41,7 @@
 #include <vector>
 
 #include "common.h"
+#include "dense.h"
 #include "internal.h"
 
 namespace pyr {
@@ -2012,6 +2013,173 @@ struct FixedMemory {
     const PyrhipBuildOutput* dst = nullptr;
 };
 
+// Whether a single build takes the dense build (dense.h): a table of a word
+// per voxel of the grid, at most 1 MiB (edge 2^6) or 64 bytes per record, which
+// is what the sorted build's buffers take. A call that names a setting other
+// than the defaults gets the kernels that the setting is about.
+bool dense_build(const PyrhipBuildTuning& tun, uint32_t log2_size, uint64_t n) {
+    if (n == 0 || log2_size > 7 || !default_tuning(tun)) return false;
+    const uint64_t slots = 1ull << (3 * log2_size);
+    return slots <= (1ull << 18) || slots <= 16 * n;
+}
+
+PyrResult run_dense(const EncodeArgs& enc, uint32_t log2_size, hipStream_t s, PyrhipBuilt* out) {
+    const uint32_t n = enc.n_old + enc.n_new;
+    const uint32_t bricks = 1u << (3 * (log2_size - 2)), nb = std::min(n, bricks);
+    // levels whose children are more than the last kernel takes, bottom first
+    struct Level {
+        uint32_t lv, parents, cap;
+        DenseLevel cells;  // of the parents
+        uint32_t *table, *owner, *slot;
+    };
+    Level wide[2];
+    uint32_t wides = 0, lv = 2;
+    for (uint32_t cells = bricks; cells > kDenseTop; cells /= 8, lv++)
+        wide[wides++] = Level{lv, cells / 8, (uint32_t)hash_cap_for(std::min(cells / 8, n), 80), {}, nullptr, nullptr, nullptr};
+    uint64_t words = 2;  // each level's parents take 2 words, plus one per child
+    for (uint64_t l = 2, c = nb, cells = bricks; l < log2_size; l++) {
+        cells /= 8;
+        const uint64_t par = std::min(c, cells);
+        words += 2 * par + c;
+        c = par;
+    }
+    const auto host_t0 = std::chrono::steady_clock::now();
+    Alloc A{{}, s};
+    // what starts at zero lies in one range: counters, look-back words, the
+    // voxel table, the hash tables
+    const uint32_t leaf_cap = (uint32_t)hash_cap_for(nb, 80);
+    const uint64_t tiles = std::max<uint64_t>(1, bricks / kDenseTile);
+    uint64_t zero = C_COUNT * 4 + tiles * 8 + (uint64_t)bricks * 256 + (uint64_t)leaf_cap * 12;
+    for (uint32_t i = 0; i < wides; i++) zero += (uint64_t)wide[i].cap * 8;
+    zero = (zero + 15) & ~15ull;
+    uint8_t* z = A.get<uint8_t>(zero);
+    DenseArgs a{};
+    a.mask = A.get<uint64_t>(bricks);
+    a.slot = A.get<uint32_t>(bricks);
+    DenseLevel brick_cells{};
+    if (wides) {
+        const uint64_t per = 3ull * bricks;
+        uint64_t all = per;
+        for (uint32_t i = 0; i < wides; i++) all += 4ull * wide[i].parents;
+        uint32_t* p = A.get<uint32_t>(all);
+        brick_cells = {p, p + bricks, p + 2ull * bricks};
+        p += per;
+        for (uint32_t i = 0; i < wides && !A.failed; i++) {
+            const uint32_t m = wide[i].parents;
+            wide[i].cells = {p, p + m, p + 2ull * m};
+            wide[i].slot = p + 3ull * m;
+            p += 4ull * m;
+        }
+    }
+    void *keys = nullptr, *attrs = nullptr, *leaves = nullptr, *nodes = nullptr;
+    const uint64_t out_bytes[4] = {(uint64_t)n * 8, (uint64_t)n * 4, (uint64_t)nb * 8, words * 4};
+    void** const outs[4] = {&keys, &attrs, &leaves, &nodes};
+    bool ok = !A.failed;
+    for (int i = 0; i < 4 && ok; i++) ok = pool_alloc(outs[i], out_bytes[i], s) == hipSuccess;
+    auto free_outputs = [&]() {
+        for (void** p : outs) pool_free(*p, s);
+    };
+    if (!ok) {
+        A.release();
+        free_outputs();
+        (void)hipGetLastError();
+        return fail(PYR_ERROR_OUT_OF_MEMORY, "device memory for a build of %u voxels", n);
+    }
+    a.old_keys = enc.old_keys;
+    a.old_vals = enc.old_vals;
+    a.n_old = enc.n_old;
+    a.voxels = enc.voxels;
+    a.n_new = enc.n_new;
+    a.log2_size = log2_size;
+    a.bricks = bricks;
+    a.leaf_cap = leaf_cap;
+    a.n_cap = n;
+    a.keys = (uint64_t*)keys;
+    a.attrs = (uint32_t*)attrs;
+    // (8-byte parts first)
+    a.status = (uint64_t*)z;
+    a.leaf_table = a.status + tiles;
+    a.counters = (uint32_t*)(a.leaf_table + leaf_cap);
+    a.table = a.counters + C_COUNT;
+    a.leaf_owner = a.table + 64ull * bricks;
+    uint32_t* zp = a.leaf_owner + leaf_cap;
+    for (uint32_t i = 0; i < wides; i++) {
+        wide[i].table = zp;
+        wide[i].owner = zp + wide[i].cap;
+        zp += 2ull * wide[i].cap;
+    }
+    const auto host_t1 = std::chrono::steady_clock::now();
+    Timer tm;
+    tm.s = s;
+    tm.mark();
+    uint32_t* const counters = a.counters;
+    uint32_t epoch = 0, launch = 0;
+    auto tile_ctr = [&]() { return counters + C_TILE + launch++; };
+    hipLaunchKernelGGL(k_dense_clear, dim3(grid_for(zero / 16, kBlock * 4, 2048)), dim3(kBlock), 0, s, (uint4*)z, zero / 16);
+    hipLaunchKernelGGL(k_dense_scatter, dim3(grid_for(n, kBlock * kDenseUnroll, 2048)), dim3(kBlock), 0, s, a);
+    tm.mark();
+    tm.mark();
+    hipLaunchKernelGGL(k_dense_voxels, dim3(grid_for(bricks, kDenseTile, 2048)), dim3(kBlock), 0, s, a, tile_ctr(), ++epoch,
+                       (uint32_t)C_ERR, (uint32_t)C_U);
+    tm.mark();
+    DenseLevel from = brick_cells;
+    if (wides)
+        hipLaunchKernelGGL(k_dense_leaves, dim3(grid_for(bricks, kBlock * kDenseItems, 2048)), dim3(kBlock), 0, s, a,
+                           brick_cells, (uint64_t*)leaves, a.status, tile_ctr(), ++epoch, (uint32_t)C_ERR,
+                           (uint32_t)C_LEAVES);
+    tm.mark();
+    for (uint32_t i = 0; i < wides; i++) {
+        const Level& w = wide[i];
+        hipLaunchKernelGGL(k_dense_insert, dim3((w.parents + kBlock - 1) / kBlock), dim3(kBlock), 0, s, from, w.parents,
+                           w.table, w.owner, w.cap, w.slot, w.cells.count, counters + C_ERR);
+        hipLaunchKernelGGL(k_dense_compact, dim3(grid_for(w.parents, kBlock, 2048)), dim3(kBlock), 0, s, from, w.cells,
+                           w.parents, w.owner, w.slot, (uint32_t*)nodes, words, a.status, tile_ctr(), ++epoch,
+                           counters + C_CUR + w.lv, counters + C_ERR);
+        from = w.cells;
+    }
+    hipLaunchKernelGGL(k_dense_top, dim3(1), dim3(kDenseTopBlock), 0, s, a, from, lv, wides ? 0u : 1u, (uint64_t*)leaves,
+                       (uint32_t*)nodes, words, counters + C_CUR + lv, (uint32_t)C_ERR, (uint32_t)C_U, (uint32_t)C_LEAVES,
+                       (uint32_t)C_ROOT, (uint32_t)C_WORDS);
+    tm.mark();
+    uint32_t c[C_TILE];
+    hipError_t e = hipMemcpyAsync(c, counters, sizeof(c), hipMemcpyDeviceToHost, s);
+    const uint64_t requested = A.requested + out_bytes[0] + out_bytes[1] + out_bytes[2] + out_bytes[3];
+    A.release();
+    const auto host_t2 = std::chrono::steady_clock::now();
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    const auto host_t3 = std::chrono::steady_clock::now();
+    if (e == hipSuccess) e = hipGetLastError();
+    if (g_timing && e == hipSuccess) {
+        using ms = std::chrono::duration<float, std::milli>;
+        std::lock_guard<std::mutex> lk(g_times_mutex);
+        g_times = PyrhipBuildTimes{};
+        g_times.encode_ms = tm.between(0, 1);
+        g_times.unique_ms = tm.between(2, 3);
+        g_times.leaves_ms = tm.between(3, 4);
+        g_times.levels_ms = tm.between(4, 5);
+        g_times.total_ms = tm.between(0, 5);
+        g_times.device_bytes = requested;
+        g_times.host_alloc_ms = ms(host_t1 - host_t0).count();
+        g_times.host_enqueue_ms = ms(host_t2 - host_t1).count();
+        g_times.host_wait_ms = ms(host_t3 - host_t2).count();
+    }
+    if (e != hipSuccess || c[C_ERR] != 0) {
+        free_outputs();
+        if (e != hipSuccess) return fail(PYR_ERROR_CUDA, "build: %s", hipGetErrorString(e));
+        return fail(PYR_ERROR_CUDA, "build: device error flags 0x%x", c[C_ERR]);
+    }
+    out->log2_size = log2_size;
+    out->root = c[C_ROOT];
+    out->nodes = (uint64_t)(uintptr_t)nodes;
+    out->node_words = c[C_WORDS];
+    out->leaves = (uint64_t)(uintptr_t)leaves;
+    out->leaf_count = c[C_LEAVES];
+    out->keys = (uint64_t)(uintptr_t)keys;
+    out->attrs = (uint64_t)(uintptr_t)attrs;
+    out->voxel_count = c[C_U];
+    return PYR_OK;
+}
+
 // One build: single geometry (enc.chunk_count == 0) or chunk batch. With
 // `gb` (batches only) the launches are captured into a graph on `s` instead
 // of run, and the buffers move to gb. With `fixed` (single builds only) no
@@ -2067,6 +2235,7 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
     const bool packed = key_bits <= 32 && rb == 8 && tun.pair_layout != 1;
     const uint32_t radix = 1u << rb;
     const uint64_t k = enc.chunk_count ? enc.chunk_count : 1;
+    if (!enc.chunk_count && !gb && !fixed && dense_build(tun, log2_size, n)) return run_dense(enc, log2_size, s, out);
 
     // upper bounds (gpu_build.zig:142-154, 291-300)
     auto cells = [&](uint32_t lv) -> uint64_t {  // cells of edge 2^lv in all chunks

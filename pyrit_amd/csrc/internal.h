@@ -54,6 +54,8 @@ void pool_free(void* p, hipStream_t s);
 // bit length of the chunk count) over the built-in defaults (tune.cpp).
 PyrhipBuildTuning resolve_tuning(const PyrhipBuildTuning* caller, uint32_t log2_size, uint32_t n,
                                  uint32_t chunk_count);
+// whether a resolved setting is the built-in default in every field
+bool default_tuning(const PyrhipBuildTuning& t);
 // whether such a build takes the bucket finish under the resolved tuning (build.hip)
 bool bucket_finish(const PyrhipBuildTuning& tun, uint32_t log2_size, uint64_t n, uint32_t chunk_count);
 

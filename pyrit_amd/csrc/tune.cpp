@@ -157,6 +157,8 @@ PyrResult measure(const Workload& w, const PyrhipBuildTuning& t, uint32_t repeat
 
 }  // namespace
 
+bool default_tuning(const PyrhipBuildTuning& t) { return same_tuning(t, kDefaults); }
+
 PyrhipBuildTuning resolve_tuning(const PyrhipBuildTuning* caller, uint32_t log2_size, uint32_t n,
                                  uint32_t chunk_count) {
     PyrhipBuildTuning t = kDefaults;

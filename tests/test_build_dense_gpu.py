@@ -1,0 +1,108 @@
+"""The dense build of small grids (a table of one word per voxel instead of
+the sort) against the oracle's arrays: every edge that takes it, both sides of
+the rule that chooses it, edits, many records of one voxel, solid grids, grids
+of one voxel, and deletions that leave nothing."""
+import numpy as np
+import pytest
+
+import oracle_py as O
+from scenes import random_points, scene_grid, grid_to_points
+from test_build_gpu import assert_same_build
+
+pytestmark = pytest.mark.gpu
+
+
+def _build(log2, pts, dense=True, old=None, **kw):
+    from pyrit_amd import gpu as g
+
+    g.set_timing(True)
+    try:
+        b = g.build(log2, pts, old=old, **kw)
+        finish = g.last_build_times()["finish"]
+    finally:
+        g.set_timing(False)
+    assert (finish == 0) == dense, finish
+    return b
+
+
+@pytest.mark.parametrize("log2", [3, 4, 5, 6, 7])
+@pytest.mark.parametrize("fill", ["rule", "full", "few"])
+def test_random_grids(hip_device, log2, fill):
+    cells = 8 ** log2
+    n = {"rule": max(2, cells // 16 + 1), "full": min(cells, 1 << 21), "few": 37}[fill]
+    pts = random_points(n, log2, seed=log2 * 7, dup_frac=0.25, delete_frac=0.05, out_frac=0.03)
+    b = _build(log2, pts, dense=cells <= 1 << 18 or 16 * len(pts) >= cells)
+    assert_same_build(b, O.gb_build(log2, pts), log2)
+
+
+def test_rule_edge(hip_device):
+    for count, dense in ((8 ** 7 // 16 - 1, False), (8 ** 7 // 16, True)):
+        pts = random_points(count, 7, seed=3, dup_frac=0.0)
+        assert_same_build(_build(7, pts, dense), O.gb_build(7, pts), 7)
+    cube = random_points(1 << 21, 8, seed=4, dup_frac=0.0)  # an edge of 2^8 never takes it
+    assert_same_build(_build(8, cube, False), O.gb_build(8, cube), 8)
+    # a named setting gets its own path, the default value of one does not change anything
+    pts = random_points(5000, 5, seed=9)
+    ref = O.gb_build(5, pts)
+    assert_same_build(_build(5, pts, False, finish=1), ref, 5)
+    assert_same_build(_build(5, pts, False, sort_items=8), ref, 5)
+    assert_same_build(_build(5, pts, True, sort_items=20), ref, 5)
+
+
+@pytest.mark.parametrize("log2,edits", [(3, 1), (5, 700), (6, 4096), (7, 311)])
+def test_edits(hip_device, log2, edits):
+    from pyrit_amd import gpu as g
+
+    size = 1 << log2
+    rng = np.random.default_rng(log2)
+    z, y, x = np.nonzero(rng.random((size, size, size)) < 0.3)
+    pts = np.zeros(len(x), O.VOXEL)
+    pts["x"], pts["y"], pts["z"], pts["attribute"] = x, y, z, rng.integers(1, 9, len(x))
+    old = g.build(log2, pts)
+    ed = random_points(edits, log2, seed=5, dup_frac=0.5, delete_frac=0.3, out_frac=0.1)
+    b = _build(log2, ed, old=old)
+    ref0 = O.gb_build(log2, pts)
+    assert_same_build(b, O.gb_build(log2, ed, ref0["keys"], ref0["attrs"]), log2)
+    # everything removed
+    gone = pts.copy()
+    gone["attribute"] = 0
+    e = _build(log2, gone, old=old)
+    assert e.voxel_count == 0 and e.nodes().tolist() == [0, 0] and e.root == 0 and e.leaf_count == 0
+
+
+def test_one_voxel_many_records(hip_device):
+    for log2 in (3, 6, 7):
+        pts = np.zeros(1 << 18, O.VOXEL)
+        pts["x"], pts["y"], pts["z"] = 5, 3, 6
+        pts["attribute"] = np.arange(1, len(pts) + 1)
+        pts["x"][::1000] = 2
+        assert_same_build(_build(log2, pts), O.gb_build(log2, pts), log2)
+        last = pts.copy()
+        last["attribute"][-1] = 0
+        assert_same_build(_build(log2, last), O.gb_build(log2, last), log2)
+
+
+@pytest.mark.parametrize("log2", [3, 5, 6, 7])
+def test_solid_and_corners(hip_device, log2):
+    n = 1 << log2
+    edge = min(n, 128)
+    solid = np.zeros(edge ** 3, O.VOXEL)
+    i = np.arange(edge ** 3)
+    solid["x"], solid["y"], solid["z"], solid["attribute"] = i % edge, i // edge % edge, i // edge // edge, 1 + i % 7
+    assert_same_build(_build(log2, solid), O.gb_build(log2, solid), log2)
+    if log2 <= 6:
+        corners = np.array([(0, 0, 0, 1), (n - 1, n - 1, n - 1, 2), (n, 0, 0, 3), (0, -1, 0, 4), (2 ** 31 - 1, 0, 0, 5),
+                            (0, 0, -2 ** 31, 6)], O.VOXEL)
+        assert_same_build(_build(log2, corners), O.gb_build(log2, corners), log2)
+        for c in corners[:2]:
+            one = np.array([c], O.VOXEL)
+            assert_same_build(_build(log2, one), O.gb_build(log2, one), log2)
+
+
+def test_scene_and_reuse(hip_device):
+    # builds of different sizes one after another reuse the cached memory
+    for log2 in (7, 5, 7, 6, 3):
+        pts = grid_to_points(scene_grid(1 << log2))
+        np.random.default_rng(log2).shuffle(pts)
+        assert_same_build(_build(log2, pts, dense=8 ** log2 <= 1 << 18 or 16 * len(pts) >= 8 ** log2),
+                          O.gb_build(log2, pts), log2)
