@@ -1742,7 +1742,7 @@ __global__ void __launch_bounds__(kLevelsBlock) k_levels_small(uint32_t* counter
 // roots of the top level and the empty geometry (gbuild.zig:607-624)
 __global__ void __launch_bounds__(kBlock) k_finalize(uint32_t* counters, uint32_t top, LevelArrays par,
                                                       uint32_t* roots, uint32_t* nodes_out, uint32_t par_cap,
-                                                      uint32_t chunk_count, uint64_t word_cap) {
+                                                      uint32_t chunk_count, uint64_t word_cap, uint32_t* host) {
     const uint32_t np = min(counters[C_NCH + top], par_cap);
     const uint32_t cur = counters[C_CUR + top];
     if (roots) {
@@ -1764,6 +1764,11 @@ __global__ void __launch_bounds__(kBlock) k_finalize(uint32_t* counters, uint32_
         counters[C_ROOT] = root;
         counters[C_WORDS] = words;
     }
+    // into the caller's pinned words: counters, roots, first voxels
+    __syncthreads();
+    if (!host) return;
+    for (uint32_t i = threadIdx.x; i < C_TILE; i += kBlock) host[i] = counters[i];
+    for (uint32_t i = threadIdx.x; i < 2 * chunk_count; i += kBlock) host[C_TILE + i] = roots[i];
 }
 
 __device__ __forceinline__ uint32_t compact3(uint64_t v) {
@@ -1876,14 +1881,55 @@ struct Alloc {
         ptrs.push_back(p);
         return p;
     }
+    // Buffers wanted together: commit() takes those of a small build as one
+    // block (freeing a block records an event: a small build's dozen blocks
+    // cost the host as much as its launches) and those of a large one each by
+    // itself, so that the cache can hand them to builds of other sizes.
+    struct Want {
+        void** p;
+        uint64_t bytes;
+    };
+    std::vector<Want> wants;
+    static constexpr uint64_t kOneBlock = 64ull << 20;
     template <class T>
-    T* get(uint64_t count) {
-        return (T*)raw(count * sizeof(T));
+    void want(T*& p, uint64_t count) {
+        p = nullptr;
+        wants.push_back({(void**)&p, count * sizeof(T)});
+    }
+    bool commit() {
+        auto aligned = [](uint64_t bytes) { return (std::max<uint64_t>(bytes, 256) + 255) & ~255ull; };
+        uint64_t total = 0;
+        for (const Want& w : wants) total += aligned(w.bytes);
+        if (base || total > kOneBlock) {
+            for (const Want& w : wants) *w.p = raw(w.bytes);
+        } else {
+            uint8_t* block = (uint8_t*)raw(total);
+            for (const Want& w : wants) {
+                if (block) *w.p = block;
+                block = block ? block + aligned(w.bytes) : nullptr;
+            }
+        }
+        wants.clear();
+        return !failed;
     }
     void release() {
         for (void* p : ptrs) pool_free(p, s);
         ptrs.clear();
     }
+};
+
+// Pinned host words that a build's last kernel writes, from the library's
+// cache of them: no copy to pageable memory, which waits for the stream and
+// is staged, is queued behind the kernels.
+struct HostWords {
+    uint32_t* p = nullptr;
+    uint64_t bytes;
+    explicit HostWords(uint64_t words) : bytes(words * 4) {
+        if (bytes) p = (uint32_t*)host_alloc(bytes);
+    }
+    ~HostWords() { host_free(p, bytes); }
+    HostWords(const HostWords&) = delete;
+    HostWords& operator=(const HostWords&) = delete;
 };
 
 // timing switch and the last build's phase times (builds may run on several
@@ -2052,29 +2098,28 @@ PyrResult run_dense(const EncodeArgs& enc, uint32_t log2_size, hipStream_t s, Py
     uint64_t zero = C_COUNT * 4 + tiles * 8 + (uint64_t)bricks * 256 + (uint64_t)leaf_cap * 12;
     for (uint32_t i = 0; i < wides; i++) zero += (uint64_t)wide[i].cap * 8;
     zero = (zero + 15) & ~15ull;
-    uint8_t* z = A.get<uint8_t>(zero);
+    uint8_t* z;
     DenseArgs a{};
-    a.mask = A.get<uint64_t>(bricks);
-    a.slot = A.get<uint32_t>(bricks);
     DenseLevel brick_cells{};
+    A.want(z, zero);
+    A.want(a.mask, bricks);
+    A.want(a.slot, bricks);
     if (wides) {
-        const uint64_t per = 3ull * bricks;
-        uint64_t all = per;
-        for (uint32_t i = 0; i < wides; i++) all += 4ull * wide[i].parents;
-        uint32_t* p = A.get<uint32_t>(all);
-        brick_cells = {p, p + bricks, p + 2ull * bricks};
-        p += per;
-        for (uint32_t i = 0; i < wides && !A.failed; i++) {
-            const uint32_t m = wide[i].parents;
-            wide[i].cells = {p, p + m, p + 2ull * m};
-            wide[i].slot = p + 3ull * m;
-            p += 4ull * m;
-        }
+        A.want(brick_cells.rep, bricks);
+        A.want(brick_cells.pos, bricks);
+        A.want(brick_cells.count, bricks);
     }
+    for (uint32_t i = 0; i < wides; i++) {
+        A.want(wide[i].cells.rep, wide[i].parents);
+        A.want(wide[i].cells.pos, wide[i].parents);
+        A.want(wide[i].cells.count, wide[i].parents);
+        A.want(wide[i].slot, wide[i].parents);
+    }
+    HostWords back(C_TILE);
     void *keys = nullptr, *attrs = nullptr, *leaves = nullptr, *nodes = nullptr;
     const uint64_t out_bytes[4] = {(uint64_t)n * 8, (uint64_t)n * 4, (uint64_t)nb * 8, words * 4};
     void** const outs[4] = {&keys, &attrs, &leaves, &nodes};
-    bool ok = !A.failed;
+    bool ok = A.commit() && back.p;
     for (int i = 0; i < 4 && ok; i++) ok = pool_alloc(outs[i], out_bytes[i], s) == hipSuccess;
     auto free_outputs = [&]() {
         for (void** p : outs) pool_free(*p, s);
@@ -2139,10 +2184,10 @@ PyrResult run_dense(const EncodeArgs& enc, uint32_t log2_size, hipStream_t s, Py
     }
     hipLaunchKernelGGL(k_dense_top, dim3(1), dim3(kDenseTopBlock), 0, s, a, from, lv, wides ? 0u : 1u, (uint64_t*)leaves,
                        (uint32_t*)nodes, words, counters + C_CUR + lv, (uint32_t)C_ERR, (uint32_t)C_U, (uint32_t)C_LEAVES,
-                       (uint32_t)C_ROOT, (uint32_t)C_WORDS);
+                       (uint32_t)C_ROOT, (uint32_t)C_WORDS, (uint32_t)C_TILE, back.p);
     tm.mark();
-    uint32_t c[C_TILE];
-    hipError_t e = hipMemcpyAsync(c, counters, sizeof(c), hipMemcpyDeviceToHost, s);
+    const uint32_t* const c = back.p;  // written by the last kernel
+    hipError_t e = hipSuccess;
     const uint64_t requested = A.requested + out_bytes[0] + out_bytes[1] + out_bytes[2] + out_bytes[3];
     A.release();
     const auto host_t2 = std::chrono::steady_clock::now();
@@ -2286,11 +2331,12 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
         A.base = fixed->base;
         A.size = fixed->size;
     }
-    uint32_t* counters = A.get<uint32_t>(C_COUNT);
+    uint32_t* counters;
+    A.want(counters, C_COUNT);
     const uint32_t segs = enc.chunk_count ? enc.chunk_count : 1;
     const uint64_t hist_words = (uint64_t)passes * segs * radix;
-    uint32_t* hist = A.get<uint32_t>(hist_words * 2);
-    uint32_t* digit_base = hist + hist_words;
+    uint32_t* hist;
+    A.want(hist, hist_words * 2);
     const uint32_t sort_tile = kBlock * sort_items;
     // record tiles: a single build has exactly ceil(n / tile); a batch's are
     // counted on the device, at most one partial tile more per chunk
@@ -2303,9 +2349,12 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
     seg.n = n;
     seg.tile = sort_tile;
     seg.off = enc.offsets;
-    uint32_t* tile_first = enc.chunk_count ? A.get<uint32_t>(enc.chunk_count + 1) : nullptr;
-    seg.desc = enc.chunk_count ? A.get<uint4>(sort_tiles) : nullptr;
-    seg.tiles = counters + C_TILES;
+    uint32_t* tile_first = nullptr;
+    uint4* tile_descs = nullptr;
+    if (enc.chunk_count) {
+        A.want(tile_first, enc.chunk_count + 1);
+        A.want(tile_descs, sort_tiles);
+    }
     const uint64_t scan_tiles = (nmax + kScanTile - 1) / kScanTile;
     // sort passes: one word per (tile, digit); unique: one per kScanTile piece of a tile
     // (sort passes: one word per tile and digit; unique/bricks: two per scan piece)
@@ -2318,28 +2367,39 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
                                                             2 * ((sort_tile + kScanTile - 1) / kScanTile)),
                            scan_tiles),
         2ull * buckets);
-    uint64_t* status = A.get<uint64_t>(status_words);
-    uint32_t* bucket_start = bucketed ? A.get<uint32_t>(buckets) : nullptr;
-    uint32_t* bucket_end = bucketed ? A.get<uint32_t>(buckets) : nullptr;
-    uint32_t* bucket_seg = bucketed && enc.chunk_count ? A.get<uint32_t>(buckets) : nullptr;
-    uint32_t* first_bucket = bucketed && enc.chunk_count ? A.get<uint32_t>(enc.chunk_count + 1) : nullptr;
-    uint32_t* status32 = narrow ? A.get<uint32_t>(sort_tiles * radix) : nullptr;
+    uint64_t* status;
+    A.want(status, status_words);
+    uint32_t *bucket_start = nullptr, *bucket_end = nullptr, *bucket_seg = nullptr, *first_bucket = nullptr;
+    uint32_t* status32 = nullptr;
+    if (bucketed) {
+        A.want(bucket_start, buckets);
+        A.want(bucket_end, buckets);
+        if (enc.chunk_count) {
+            A.want(bucket_seg, buckets);
+            A.want(first_bucket, enc.chunk_count + 1);
+        }
+    }
+    if (narrow) A.want(status32, sort_tiles * radix);
     // pass 0 counted by encode (8-bit digits): per-tile run prefixes and per-run totals
     const uint32_t eblocks = (uint32_t)std::min<uint64_t>(sort_tiles, 2048);
     const uint32_t per_block = (uint32_t)((sort_tiles + eblocks - 1) / eblocks);
     const bool counted = radix == (uint32_t)kBlock && tun.counted_pass != 2;
-    uint32_t* tile_run = counted ? A.get<uint32_t>(sort_tiles * radix) : nullptr;
-    uint32_t* run_sum = counted ? A.get<uint32_t>((uint64_t)eblocks * radix * 2) : nullptr;
-    uint64_t* brick_key = A.get<uint64_t>(nb);
-    uint64_t* masks = A.get<uint64_t>(nb);
+    uint32_t *tile_run = nullptr, *run_sum = nullptr;
+    if (counted) {
+        A.want(tile_run, sort_tiles * radix);
+        A.want(run_sum, (uint64_t)eblocks * radix * 2);
+    }
+    uint64_t *brick_key, *masks;
+    A.want(brick_key, nb);
+    A.want(masks, nb);
     uint64_t* table = nullptr;
     uint32_t* owner = nullptr;
     uint32_t* slot = nullptr;
     LevelArrays set[2];
     uint32_t* node_tmp = nullptr;
     uint32_t* node_len = nullptr;
-    uint32_t* roots_dev = enc.chunk_count ? A.get<uint32_t>(enc.chunk_count * 2) : nullptr;
-    uint32_t* first_dev = enc.chunk_count ? roots_dev + enc.chunk_count : nullptr;
+    uint32_t* roots_dev = nullptr;
+    if (enc.chunk_count) A.want(roots_dev, enc.chunk_count * 2);
     // caller-owned outputs; of the two key/value buffer pairs one ends up
     // holding the unique voxels (Built.keys/attrs), the other is freed
     uint64_t* kb[2] = {nullptr, nullptr};
@@ -2358,24 +2418,37 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
         if (q == 0 || !packed) out_ok &= out_alloc((void**)&vb[q], (uint64_t)nmax * 4);
     }
     // the buffers sized by the brick count, the leaves and node words among them
+    // (commits what is wanted, the buffers above included when they still are)
     auto alloc_levels = [&]() {
         bool ok = true;
-        table = A.get<uint64_t>(lz.cap);
-        owner = A.get<uint32_t>(lz.cap);
-        slot = A.get<uint32_t>(lz.nb);
+        A.want(table, lz.cap);
+        A.want(owner, lz.cap);
+        A.want(slot, lz.nb);
         for (int q = 0; q < 2; q++) {
-            set[q].key = q == 0 ? brick_key : A.get<uint64_t>(lz.np2);
-            set[q].rep = A.get<uint32_t>(q == 0 ? lz.nb : lz.np2);
-            set[q].pos = A.get<uint32_t>(q == 0 ? lz.nb : lz.np2);
-            set[q].count = A.get<uint32_t>(q == 0 ? lz.nb : lz.np2);
+            if (q) A.want(set[q].key, lz.np2);
+            A.want(set[q].rep, q == 0 ? lz.nb : lz.np2);
+            A.want(set[q].pos, q == 0 ? lz.nb : lz.np2);
+            A.want(set[q].count, q == 0 ? lz.nb : lz.np2);
         }
-        node_tmp = A.get<uint32_t>(lz.np2 * kNodeStride);
-        node_len = A.get<uint32_t>(lz.np2);
+        A.want(node_tmp, lz.np2 * kNodeStride);
+        A.want(node_len, lz.np2);
+        ok &= A.commit();
         ok &= out_alloc((void**)&leaves_out, lz.nb * 8);
         ok &= out_alloc((void**)&nodes_out, lz.words * 4);
-        return ok && !A.failed;
+        set[0].key = brick_key;
+        return ok;
     };
-    if (!exact_levels) out_ok &= alloc_levels();
+    if (exact_levels) out_ok &= A.commit();
+    else out_ok &= alloc_levels();
+    uint32_t* const digit_base = hist + hist_words;
+    uint32_t* const first_dev = enc.chunk_count ? roots_dev + enc.chunk_count : nullptr;
+    seg.desc = tile_descs;
+    seg.tiles = counters + C_TILES;
+    // the read-back: pinned words that the last kernel writes
+    // (a build without allocation copies them into `local` instead)
+    HostWords back(gb || fixed ? 0 : C_TILE + 2ull * enc.chunk_count);
+    uint32_t local[C_TILE];
+    out_ok &= gb || fixed || back.p;
     auto free_outputs = [&]() {
         if (fixed) return;
         for (int q = 0; q < 2; q++) {
@@ -2581,22 +2654,14 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
         ch ^= 1;
     }
     hipLaunchKernelGGL(k_finalize, dim3(1), dim3(kBlock), 0, s, counters, log2_size, set[ch], roots_dev,
-                       nodes_out, (uint32_t)std::min(set_cap[ch], lz.np2), enc.chunk_count, lz.words);
+                       nodes_out, (uint32_t)std::min(set_cap[ch], lz.np2), enc.chunk_count, lz.words,
+                       gb ? gb->host : back.p);
     tm.mark();
 
-    // single read-back (gpu_build.zig:338-344); a graph copies into its pinned buffer
-    uint32_t c[C_TILE];
-    uint32_t* const hc = gb ? gb->host : c;
-    if (gb) {
-        roots_host = gb->host + C_TILE;
-        first_host = roots_host + enc.chunk_count;
-    }
-    hipError_t e = hipMemcpyAsync(hc, counters, sizeof(c), hipMemcpyDeviceToHost, s);
-    if (enc.chunk_count && e == hipSuccess) {
-        e = hipMemcpyAsync(roots_host, roots_dev, enc.chunk_count * 4, hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(first_host, first_dev, enc.chunk_count * 4, hipMemcpyDeviceToHost, s);
-    }
+    // single read-back (gpu_build.zig:338-344): pinned words, a graph's own
+    const uint32_t* const c = gb ? gb->host : fixed ? local : back.p;
+    hipError_t e = hipSuccess;
+    if (fixed) e = hipMemcpyAsync(local, counters, sizeof(local), hipMemcpyDeviceToHost, s);
     if (gb) {
         hipGraph_t graph = nullptr;
         const hipError_t ce = hipStreamEndCapture(s, &graph);
@@ -2627,6 +2692,10 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     const auto host_t3 = std::chrono::steady_clock::now();
     if (e == hipSuccess) e = hipGetLastError();
+    if (enc.chunk_count && e == hipSuccess) {
+        memcpy(roots_host, c + C_TILE, enc.chunk_count * 4ull);
+        memcpy(first_host, c + C_TILE + enc.chunk_count, enc.chunk_count * 4ull);
+    }
     if (g_timing && !fixed && e == hipSuccess) {
         std::lock_guard<std::mutex> lk(g_times_mutex);
         g_times.encode_ms = tm.between(0, 1);

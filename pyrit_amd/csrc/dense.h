@@ -380,7 +380,7 @@ __global__ void __launch_bounds__(kDenseTopBlock) k_dense_top(DenseArgs a, Dense
                                                                uint64_t* leaves_out, uint32_t* nodes_out,
                                                                uint64_t word_cap, const uint32_t* cursor, uint32_t c_err,
                                                                uint32_t c_unique, uint32_t c_leaves, uint32_t c_root,
-                                                               uint32_t c_words) {
+                                                               uint32_t c_words, uint32_t counts, uint32_t* host) {
     __shared__ uint32_t s_ref[kDenseTop], s_cnt[kDenseTop];
     __shared__ uint32_t s_pos[kDenseTop];
     __shared__ uint32_t s_hash[kDenseTopHash], s_owner[kDenseTopHash];
@@ -480,6 +480,9 @@ __global__ void __launch_bounds__(kDenseTopBlock) k_dense_top(DenseArgs a, Dense
         a.counters[c_root] = root;
         a.counters[c_words] = cur;
     }
+    // the counters into the caller's pinned words
+    __syncthreads();
+    if (tid < counts) host[tid] = a.counters[tid];
 }
 
 }  // namespace pyr

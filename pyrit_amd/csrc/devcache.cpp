@@ -156,11 +156,72 @@ void pool_free(void* p, hipStream_t s) {
     if (c.free_bytes > c.limit) trim_locked(c, c.limit);
 }
 
+namespace {
+struct HostCache {
+    std::mutex m;
+    std::multimap<uint64_t, void*> free_blocks;  // class -> block
+    uint64_t free_bytes = 0;
+};
+HostCache& host_cache() {
+    static HostCache* c = new HostCache();
+    return *c;
+}
+constexpr uint64_t kHostCacheLimit = 1ull << 20;
+uint64_t host_class(uint64_t bytes) {
+    uint64_t c = 1024;
+    while (c < bytes) c <<= 1;
+    return c;
+}
+}  // namespace
+
+void* host_alloc(uint64_t bytes) {
+    const uint64_t cls = host_class(bytes);
+    HostCache& c = host_cache();
+    {
+        std::lock_guard<std::mutex> lk(c.m);
+        auto it = c.free_blocks.find(cls);
+        if (it != c.free_blocks.end()) {
+            void* p = it->second;
+            c.free_blocks.erase(it);
+            c.free_bytes -= cls;
+            return p;
+        }
+    }
+    void* p = nullptr;
+    if (hipHostMalloc(&p, cls, hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return p;
+}
+
+void host_free(void* p, uint64_t bytes) {
+    if (!p) return;
+    const uint64_t cls = host_class(bytes);
+    HostCache& c = host_cache();
+    {
+        std::lock_guard<std::mutex> lk(c.m);
+        if (c.free_bytes + cls <= kHostCacheLimit) {
+            c.free_blocks.emplace(cls, p);
+            c.free_bytes += cls;
+            return;
+        }
+    }
+    (void)hipHostFree(p);
+}
+
 }  // namespace pyr
 
 extern "C" {
 
 PYR_API void pyrhip_trim(void) {
+    {
+        pyr::HostCache& h = pyr::host_cache();
+        std::lock_guard<std::mutex> lk(h.m);
+        for (auto& b : h.free_blocks) (void)hipHostFree(b.second);
+        h.free_blocks.clear();
+        h.free_bytes = 0;
+    }
     pyr::Cache& c = pyr::cache();
     std::lock_guard<std::mutex> lk(c.m);
     pyr::trim_locked(c, 0);

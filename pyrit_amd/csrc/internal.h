@@ -47,6 +47,10 @@ inline PyrResult fail(PyrResult code, const char* fmt, ...) {
 // stay mapped and serve later requests of their size class, reuse on another
 // stream waits for the freeing stream on the device.
 hipError_t pool_alloc(void** p, uint64_t bytes, hipStream_t s);
+// Pinned host memory that kernels write, cached (at most 1 MiB of free
+// blocks); host_free after the stream that used it has been waited for.
+void* host_alloc(uint64_t bytes);
+void host_free(void* p, uint64_t bytes);
 void pool_free(void* p, hipStream_t s);
 
 // Build tuning of one workload: the caller's non-zero fields over the
