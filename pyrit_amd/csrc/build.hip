@@ -38,6 +38,7 @@
 #include <mutex>
 #include <new>
 #include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "common.h"
@@ -2024,6 +2025,14 @@ void launch_unique_bricks(hipStream_t s, uint32_t items, uint32_t sort_tile, uin
 
 }  // namespace
 
+// Cells of the lowest dense level of a build that is not dense throughout: a
+// dense level costs two launches of a few microseconds that read its cells
+// in order, a general one four of which k_level_build alone takes 36 us however
+// few its elements. Builds with the dense levels from 2^12, 2^15, 2^18 and 2^21
+// cells (and without): 2^9 terrain 2152, 2119, 2063, 2024 (2260) us, 2^11
+// surface 1500, 1428, 1378, 1473 (1562), 48 chunks 1609, 1577, 1503, 1587 (1648).
+constexpr uint64_t kDenseCells = 1ull << 18;
+
 // A chunk-batch build captured into a HIP graph (pyrhip_graph_*): every
 // buffer is allocated once for the largest batch, the kernels take their
 // sizes from the device arrays (offsets, counters), and a replay ends with
@@ -2069,19 +2078,67 @@ bool dense_build(const PyrhipBuildTuning& tun, uint32_t log2_size, uint64_t n) {
     return slots <= (1ull << 18) || slots <= 16 * n;
 }
 
+// Dense levels (dense.h) from `cells` cells on level lv up to the one that
+// k_dense_top starts from.
+struct DenseLevels {
+    struct Wide {
+        uint32_t lv, parents, cap;
+        DenseLevel cells{};  // of the parents
+        uint32_t *table = nullptr, *owner = nullptr, *slot = nullptr;
+    };
+    Wide wide[4];
+    uint32_t wides = 0, top = 0;  // top: k_dense_top's level
+    // elements: no level has more (bricks or records)
+    DenseLevels(uint32_t lv, uint64_t cells, uint64_t elements) {
+        for (; cells > kDenseTop; cells /= 8, lv++)
+            wide[wides++] = Wide{lv, (uint32_t)(cells / 8), (uint32_t)hash_cap_for(std::min<uint64_t>(cells / 8, elements), 80)};
+        top = lv;
+    }
+    uint64_t zero_words() const {  // hash tables and owners
+        uint64_t w = 0;
+        for (uint32_t i = 0; i < wides; i++) w += 2ull * wide[i].cap;
+        return w;
+    }
+    void want(Alloc& A) {
+        for (uint32_t i = 0; i < wides; i++) {
+            A.want(wide[i].cells.rep, wide[i].parents);
+            A.want(wide[i].cells.pos, wide[i].parents);
+            A.want(wide[i].cells.count, wide[i].parents);
+            A.want(wide[i].slot, wide[i].parents);
+        }
+    }
+    void zeroed(uint32_t* p) {
+        for (uint32_t i = 0; i < wides; i++) {
+            wide[i].table = p;
+            wide[i].owner = p + wide[i].cap;
+            p += 2ull * wide[i].cap;
+        }
+    }
+    // the launches; `next` gives each scan its tile counter and epoch
+    template <typename Next>
+    void launch(hipStream_t s, DenseArgs a, DenseLevel from, bool bricks, const DenseChunks& chunks, uint64_t* leaves,
+                uint32_t* nodes, uint64_t words, Next next, uint32_t* host) const {
+        uint32_t* const counters = a.counters;
+        for (uint32_t i = 0; i < wides; i++) {
+            const Wide& w = wide[i];
+            hipLaunchKernelGGL(k_dense_insert, dim3((w.parents + kBlock - 1) / kBlock), dim3(kBlock), 0, s, from, w.lv,
+                               chunks, w.parents, w.table, w.owner, w.cap, w.slot, w.cells.count, counters + C_ERR);
+            const auto t = next();
+            hipLaunchKernelGGL(k_dense_compact, dim3(grid_for(w.parents, kBlock, 2048)), dim3(kBlock), 0, s, from,
+                               w.cells, w.parents, w.owner, w.slot, nodes, words, a.status, t.first, t.second,
+                               counters + C_CUR + w.lv, counters + C_ERR);
+            from = w.cells;
+        }
+        hipLaunchKernelGGL(k_dense_top, dim3(1), dim3(kDenseTopBlock), 0, s, a, from, top, bricks ? 1u : 0u, chunks,
+                           leaves, nodes, words, counters + C_CUR + top, (uint32_t)C_ERR, (uint32_t)C_U,
+                           (uint32_t)C_LEAVES, (uint32_t)C_ROOT, (uint32_t)C_WORDS, (uint32_t)C_TILE, host);
+    }
+};
+
 PyrResult run_dense(const EncodeArgs& enc, uint32_t log2_size, hipStream_t s, PyrhipBuilt* out) {
     const uint32_t n = enc.n_old + enc.n_new;
     const uint32_t bricks = 1u << (3 * (log2_size - 2)), nb = std::min(n, bricks);
-    // levels whose children are more than the last kernel takes, bottom first
-    struct Level {
-        uint32_t lv, parents, cap;
-        DenseLevel cells;  // of the parents
-        uint32_t *table, *owner, *slot;
-    };
-    Level wide[2];
-    uint32_t wides = 0, lv = 2;
-    for (uint32_t cells = bricks; cells > kDenseTop; cells /= 8, lv++)
-        wide[wides++] = Level{lv, cells / 8, (uint32_t)hash_cap_for(std::min(cells / 8, n), 80), {}, nullptr, nullptr, nullptr};
+    DenseLevels levels(2, bricks, n);
     uint64_t words = 2;  // each level's parents take 2 words, plus one per child
     for (uint64_t l = 2, c = nb, cells = bricks; l < log2_size; l++) {
         cells /= 8;
@@ -2096,25 +2153,19 @@ PyrResult run_dense(const EncodeArgs& enc, uint32_t log2_size, hipStream_t s, Py
     const uint32_t leaf_cap = (uint32_t)hash_cap_for(nb, 80);
     const uint64_t tiles = std::max<uint64_t>(1, bricks / kDenseTile);
     uint64_t zero = C_COUNT * 4 + tiles * 8 + (uint64_t)bricks * 256 + (uint64_t)leaf_cap * 12;
-    for (uint32_t i = 0; i < wides; i++) zero += (uint64_t)wide[i].cap * 8;
-    zero = (zero + 15) & ~15ull;
+    zero = (zero + levels.zero_words() * 4 + 15) & ~15ull;
     uint8_t* z;
     DenseArgs a{};
     DenseLevel brick_cells{};
     A.want(z, zero);
     A.want(a.mask, bricks);
     A.want(a.slot, bricks);
-    if (wides) {
+    if (levels.wides) {
         A.want(brick_cells.rep, bricks);
         A.want(brick_cells.pos, bricks);
         A.want(brick_cells.count, bricks);
     }
-    for (uint32_t i = 0; i < wides; i++) {
-        A.want(wide[i].cells.rep, wide[i].parents);
-        A.want(wide[i].cells.pos, wide[i].parents);
-        A.want(wide[i].cells.count, wide[i].parents);
-        A.want(wide[i].slot, wide[i].parents);
-    }
+    levels.want(A);
     HostWords back(C_TILE);
     void *keys = nullptr, *attrs = nullptr, *leaves = nullptr, *nodes = nullptr;
     const uint64_t out_bytes[4] = {(uint64_t)n * 8, (uint64_t)n * 4, (uint64_t)nb * 8, words * 4};
@@ -2147,12 +2198,7 @@ PyrResult run_dense(const EncodeArgs& enc, uint32_t log2_size, hipStream_t s, Py
     a.counters = (uint32_t*)(a.leaf_table + leaf_cap);
     a.table = a.counters + C_COUNT;
     a.leaf_owner = a.table + 64ull * bricks;
-    uint32_t* zp = a.leaf_owner + leaf_cap;
-    for (uint32_t i = 0; i < wides; i++) {
-        wide[i].table = zp;
-        wide[i].owner = zp + wide[i].cap;
-        zp += 2ull * wide[i].cap;
-    }
+    levels.zeroed(a.leaf_owner + leaf_cap);
     const auto host_t1 = std::chrono::steady_clock::now();
     Timer tm;
     tm.s = s;
@@ -2167,24 +2213,13 @@ PyrResult run_dense(const EncodeArgs& enc, uint32_t log2_size, hipStream_t s, Py
     hipLaunchKernelGGL(k_dense_voxels, dim3(grid_for(bricks, kDenseTile, 2048)), dim3(kBlock), 0, s, a, tile_ctr(), ++epoch,
                        (uint32_t)C_ERR, (uint32_t)C_U);
     tm.mark();
-    DenseLevel from = brick_cells;
-    if (wides)
+    if (levels.wides)
         hipLaunchKernelGGL(k_dense_leaves, dim3(grid_for(bricks, kBlock * kDenseItems, 2048)), dim3(kBlock), 0, s, a,
                            brick_cells, (uint64_t*)leaves, a.status, tile_ctr(), ++epoch, (uint32_t)C_ERR,
                            (uint32_t)C_LEAVES);
     tm.mark();
-    for (uint32_t i = 0; i < wides; i++) {
-        const Level& w = wide[i];
-        hipLaunchKernelGGL(k_dense_insert, dim3((w.parents + kBlock - 1) / kBlock), dim3(kBlock), 0, s, from, w.parents,
-                           w.table, w.owner, w.cap, w.slot, w.cells.count, counters + C_ERR);
-        hipLaunchKernelGGL(k_dense_compact, dim3(grid_for(w.parents, kBlock, 2048)), dim3(kBlock), 0, s, from, w.cells,
-                           w.parents, w.owner, w.slot, (uint32_t*)nodes, words, a.status, tile_ctr(), ++epoch,
-                           counters + C_CUR + w.lv, counters + C_ERR);
-        from = w.cells;
-    }
-    hipLaunchKernelGGL(k_dense_top, dim3(1), dim3(kDenseTopBlock), 0, s, a, from, lv, wides ? 0u : 1u, (uint64_t*)leaves,
-                       (uint32_t*)nodes, words, counters + C_CUR + lv, (uint32_t)C_ERR, (uint32_t)C_U, (uint32_t)C_LEAVES,
-                       (uint32_t)C_ROOT, (uint32_t)C_WORDS, (uint32_t)C_TILE, back.p);
+    levels.launch(s, a, brick_cells, !levels.wides, DenseChunks{nullptr, nullptr, 1, log2_size}, (uint64_t*)leaves,
+                  (uint32_t*)nodes, words, [&]() { return std::make_pair(tile_ctr(), ++epoch); }, back.p);
     tm.mark();
     const uint32_t* const c = back.p;  // written by the last kernel
     hipError_t e = hipSuccess;
@@ -2365,7 +2400,7 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
     const uint64_t status_words = std::max<uint64_t>(
         std::max<uint64_t>(sort_tiles * std::max<uint32_t>(narrow ? 0u : radix,
                                                             2 * ((sort_tile + kScanTile - 1) / kScanTile)),
-                           scan_tiles),
+                           std::max<uint64_t>(scan_tiles, kDenseCells / (8 * kBlock))),
         2ull * buckets);
     uint64_t* status;
     A.want(status, status_words);
@@ -2395,6 +2430,20 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
     uint64_t* table = nullptr;
     uint32_t* owner = nullptr;
     uint32_t* slot = nullptr;
+    // the levels from lv0 up are dense (dense.h) when their cells are few (16
+    // bytes each: at most 8 per record beyond those of the last kernel): all
+    // of them, or those above the levels of a build with more bricks than one
+    // workgroup takes
+    uint32_t lv0 = 2;
+    const uint64_t cells_max = std::min<uint64_t>(kDenseCells, std::max<uint64_t>(kDenseTop, nmax / 2));
+    while (lv0 < log2_size && (k << (3 * (log2_size - lv0))) > cells_max) lv0++;
+    const uint64_t dense_cells = k << (3 * (log2_size - lv0));
+    const bool dense_levels = tun.levels == 0 && !fixed && k <= kDenseTop && (lv0 == 2 || nb > kLevelsSmallBricks);
+    if (!dense_levels) lv0 = log2_size;
+    DenseLevels dense(lv0, dense_levels ? dense_cells : 0, nmax);
+    DenseLevel dense_from{};  // the cells of level lv0
+    uint32_t* dense_zero = nullptr;
+    const uint64_t dense_words = (dense_cells + dense.zero_words() + 3) & ~3ull;
     LevelArrays set[2];
     uint32_t* node_tmp = nullptr;
     uint32_t* node_len = nullptr;
@@ -2432,10 +2481,18 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
         }
         A.want(node_tmp, lz.np2 * kNodeStride);
         A.want(node_len, lz.np2);
+        if (dense_levels) {
+            A.want(dense_from.rep, dense_cells);
+            A.want(dense_from.pos, dense_cells);
+            A.want(dense_zero, dense_words);
+            dense.want(A);
+        }
         ok &= A.commit();
         ok &= out_alloc((void**)&leaves_out, lz.nb * 8);
         ok &= out_alloc((void**)&nodes_out, lz.words * 4);
         set[0].key = brick_key;
+        dense_from.count = dense_zero;
+        if (ok && dense_levels) dense.zeroed(dense_zero + dense_cells);
         return ok;
     };
     if (exact_levels) out_ok &= A.commit();
@@ -2597,11 +2654,11 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
                            leaves_out, set[0].rep, set[0].pos, (uint32_t)lz.nb);
     }
     tm.mark();
-    // 5. node levels: one workgroup and one launch for small builds, else
-    // four launches per level
+    // 5. node levels: four launches per level, then the dense ones; a build of
+    // few bricks in a large grid in one workgroup and one launch
     int ch = 0;
     const uint64_t set_cap[2] = {lz.nb, lz.np2};
-    const bool small_levels = tun.levels == 2 || (tun.levels == 0 && lz.nb <= kLevelsSmallBricks);
+    const bool small_levels = !dense_levels && (tun.levels == 2 || (tun.levels == 0 && lz.nb <= kLevelsSmallBricks));
     if (small_levels && log2_size > 2) {
         LevelArgs la{};
         la.chunk_log2 = enc.chunk_log2;
@@ -2621,7 +2678,7 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
                            (uint32_t)set_cap[0], (uint32_t)set_cap[1], (uint32_t)lz.np2, nodes_out);
         ch = (log2_size - 2) & 1;
     }
-    for (uint32_t lv = 2; lv < log2_size && !small_levels; lv++) {
+    for (uint32_t lv = 2; lv < lv0 && !small_levels; lv++) {
         LevelArgs la{};
         la.lv = lv;
         la.top_shift = 3 * (log2_size - lv);
@@ -2653,9 +2710,24 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
                            dim3(kBlock), 0, s, sc2, la, nodes_out);
         ch ^= 1;
     }
-    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(kBlock), 0, s, counters, log2_size, set[ch], roots_dev,
-                       nodes_out, (uint32_t)std::min(set_cap[ch], lz.np2), enc.chunk_count, lz.words,
-                       gb ? gb->host : back.p);
+    if (dense_levels) {
+        hipLaunchKernelGGL(k_dense_clear, dim3(grid_for(dense_words / 4, kBlock * 4, 2048)), dim3(kBlock), 0, s,
+                           (uint4*)dense_zero, dense_words / 4);
+        const uint64_t elements = std::min<uint64_t>(set_cap[ch], dense_cells);
+        hipLaunchKernelGGL(k_dense_spread, dim3(grid_for(elements, kBlock, 2048)), dim3(kBlock), 0, s, counters,
+                           (uint32_t)(C_NCH + lv0), (uint32_t)set_cap[ch], set[ch].key, set[ch].rep, set[ch].pos,
+                           set[ch].count, dense_from, (uint32_t)dense_cells, counters + C_ERR);
+        DenseArgs da{};
+        da.log2_size = log2_size;
+        da.counters = counters;
+        da.status = status;
+        dense.launch(s, da, dense_from, false, DenseChunks{enc.chunk_log2, roots_dev, (uint32_t)k, log2_size}, leaves_out,
+                     nodes_out, lz.words, [&]() { return std::make_pair(tile_ctr(), ++epoch); },
+                     gb ? gb->host : back.p);
+    } else {
+        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(kBlock), 0, s, counters, log2_size, set[ch], roots_dev, nodes_out,
+                           (uint32_t)std::min(set_cap[ch], lz.np2), enc.chunk_count, lz.words, gb ? gb->host : back.p);
+    }
     tm.mark();
 
     // single read-back (gpu_build.zig:338-344): pinned words, a graph's own

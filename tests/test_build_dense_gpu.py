@@ -106,3 +106,43 @@ def test_scene_and_reuse(hip_device):
         np.random.default_rng(log2).shuffle(pts)
         assert_same_build(_build(log2, pts, dense=8 ** log2 <= 1 << 18 or 16 * len(pts) >= 8 ** log2),
                           O.gb_build(log2, pts), log2)
+
+
+@pytest.mark.parametrize("log2,count,mixed", [(3, 1, False), (6, 1, True), (5, 3, True), (8, 3, True), (7, 65, True),
+                                              (8, 64, True), (4, 513, True), (3, 4096, False), (3, 4097, False),
+                                              (9, 5, False)])
+def test_batch_levels(hip_device, log2, count, mixed):
+    """Batches whose upper levels are dense, from all levels to none: chunks
+    that end on every level, empty chunks, and counts around the last kernel's
+    cells."""
+    from pyrit_amd import gpu as g
+
+    rng = np.random.default_rng(count)
+    l2 = rng.integers(3, log2 + 1, count).astype(np.uint8) if mixed else None
+    chunks = []
+    for c in range(count):
+        edge = int(l2[c]) if mixed else log2
+        n = 0 if c % 7 == 3 else int(rng.integers(1, min(8 ** edge, 200000 // count + 40)))
+        chunks.append(random_points(n, edge, int(rng.integers(1 << 30)), dup_frac=0.1, delete_frac=0.02) if n else
+                      np.zeros(0, O.VOXEL))
+    offs = np.concatenate([[0], np.cumsum([len(c) for c in chunks])]).astype(np.uint32)
+    vox = np.concatenate(chunks)
+    ref, rroots, rfirst = O.gb_build_chunks(log2, vox, offs, l2)
+    for levels in (0, 1, 2):
+        b, roots, first = g.build_chunks(log2, vox, offs, l2, levels=levels)
+        assert_same_build(b, ref, log2)
+        assert np.array_equal(roots, rroots) and np.array_equal(first, rfirst)
+
+
+@pytest.mark.parametrize("log2,n", [(7, 40000), (8, 300000), (9, 40000), (10, 600000), (13, 50000)])
+def test_upper_levels(hip_device, log2, n):
+    from pyrit_amd import gpu as g
+
+    pts = random_points(n, log2, seed=n, dup_frac=0.1, delete_frac=0.02)
+    ref = O.gb_build(log2, pts)
+    for levels in (0, 1):
+        assert_same_build(g.build(log2, pts, levels=levels), ref, log2)
+    one = pts[:1].copy()
+    one["x"] = one["y"] = one["z"] = (1 << log2) - 1
+    many = np.repeat(one, 70000)  # one voxel of many records in a large grid
+    assert_same_build(g.build(log2, many), O.gb_build(log2, many), log2)
