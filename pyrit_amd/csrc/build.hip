@@ -235,6 +235,19 @@ __device__ __forceinline__ void encode_one(const EncodeArgs& a, int32_t n, uint3
     }
 }
 
+// the same with a 32-bit key
+__device__ __forceinline__ void encode_one(const EncodeArgs& a, int32_t n, uint32_t i, int4 v, uint32_t& key,
+                                           uint32_t& val) {
+    if (i < a.n_old) {
+        key = (uint32_t)a.old_keys[i];
+        val = a.old_vals[i];
+        return;
+    }
+    const bool in = (uint32_t)v.x < (uint32_t)n && (uint32_t)v.y < (uint32_t)n && (uint32_t)v.z < (uint32_t)n;
+    key = in ? local_key32((uint32_t)v.x, (uint32_t)v.y, (uint32_t)v.z) : 1u << local_bits(a.log2_size);
+    val = in ? (uint32_t)v.w : 0u;
+}
+
 constexpr int kEncodeUnroll = 4;  // records per thread whose loads are in flight together
 
 // Records of a contiguous run of tiles per block, plus the digit histograms
@@ -247,10 +260,11 @@ constexpr int kEncodeUnroll = 4;  // records per thread whose loads are in fligh
 // serialised ones on the same bin. (Matching up to four digits of a wave
 // this way made the 1024^3 encode 19 % slower, and a second digit alone 3 %:
 // the matching costs more VALU work per record than the serialised atomics.)
+template <typename K>
 __device__ __forceinline__ void emit_record(const EncodeArgs& a, uint32_t* s_hist, uint32_t radix, uint32_t i,
-                                            uint64_t key, uint32_t val) {
-    if (a.packed) {
-        __builtin_nontemporal_store((key << 32) | val, &a.keys[i]);
+                                            K key, uint32_t val) {
+    if (sizeof(K) == 4 || a.packed) {
+        __builtin_nontemporal_store(((uint64_t)key << 32) | val, &a.keys[i]);
     } else {
         a.keys[i] = key;
         a.vals[i] = val;
@@ -269,6 +283,11 @@ __device__ __forceinline__ void emit_record(const EncodeArgs& a, uint32_t* s_his
     }
 }
 
+// K: 32-bit keys for packed records of grids up to 2^10, 64 bits otherwise: the
+// 64-bit spreading of the coordinates was most of the kernel's vector work
+// (1024^3 grid, 5.1e8 records: 2.87 -> 2.38 ms, 5.1 TB/s; the copy probe reaches
+// 5.5).
+template <typename K>
 __global__ void __launch_bounds__(kBlock) k_encode(EncodeArgs a, Segs g, uint32_t tiles_per_block) {
     extern __shared__ uint32_t s_hist[];
     const uint32_t radix = 1u << a.radix_bits, bins = a.passes * radix;
@@ -317,7 +336,7 @@ __global__ void __launch_bounds__(kBlock) k_encode(EncodeArgs a, Segs g, uint32_
             for (int u = 0; u < kEncodeUnroll; u++) {
                 const uint32_t j = j0 + u * kBlock + threadIdx.x;
                 if (j < d.z) {
-                    uint64_t key;
+                    K key;
                     uint32_t val;
                     encode_one(a, edge, d.y + j, raw[u], key, val);
                     emit_record(a, s_hist, radix, d.y + j, key, val);
@@ -468,6 +487,11 @@ __global__ void __launch_bounds__(kBlock) k_sort_pass(SortArgs a) {
     uint64_t* keys_out = a.b.keys[src ^ 1];
     uint32_t* vals_out = a.b.vals[src ^ 1];
     const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
+    // (a packed record's digit lies in its high word: one 32-bit extract)
+    auto digit = [&](uint64_t key) -> uint32_t {
+        if constexpr (PACKED) return __builtin_amdgcn_ubfe((uint32_t)(key >> 32), a.shift - 32, RB);
+        else return (uint32_t)(key >> a.shift) & (R - 1);
+    };
     // per-wave lane masks of each digit while ranking one row (zero between
     // rows); the staging area is free until the ranking is done
     // (wider digits whose masks do not fit match the digit with RB ballots)
@@ -511,7 +535,7 @@ __global__ void __launch_bounds__(kBlock) k_sort_pass(SortArgs a) {
 #pragma unroll
     for (int i = 0; i < kSortItems; i++) {
         bool ok = wbase + i * kWave + lane < count;
-        uint32_t d = (uint32_t)(k[i] >> a.shift) & (R - 1);
+        uint32_t d = digit(k[i]);
         uint64_t peers = 0;
         if constexpr (kLdsMatch) {
             uint64_t rest = __ballot(ok);
@@ -619,7 +643,7 @@ __global__ void __launch_bounds__(kBlock) k_sort_pass(SortArgs a) {
 #pragma unroll
     for (int i = 0; i < kSortItems; i++) {
         if (wbase + i * kWave + lane < count) {
-            uint32_t d = (uint32_t)(k[i] >> a.shift) & (R - 1);
+            uint32_t d = digit(k[i]);
             uint32_t pos = s_local[d] + s_wave_cnt[wave][d] + rank[i];
             s_keys[pos] = k[i];
             if constexpr (!PACKED) s_vals[pos] = v[i];
@@ -684,7 +708,7 @@ __global__ void __launch_bounds__(kBlock) k_sort_pass(SortArgs a) {
     // coalesced write-out: consecutive slots of one digit are consecutive in HBM
     for (uint32_t j = tid; j < count; j += kBlock) {
         uint64_t key = s_keys[j];
-        uint32_t d = (uint32_t)(key >> a.shift) & (R - 1);
+        uint32_t d = digit(key);
         uint64_t dst = s_dst[d] + (j - s_local[d]);
         if (dst >= a.g.n) {  // only after a failed look-back
             atomicOr(a.err, 16u);
@@ -2566,8 +2590,11 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
         }
         enc.tile_run = tile_run;
         enc.run_sum = run_sum;
-        hipLaunchKernelGGL(k_encode, dim3(eblocks), dim3(kBlock), passes * radix * sizeof(uint32_t), s, enc, seg,
-                           per_block);
+        const uint32_t hist_bytes = passes * radix * sizeof(uint32_t);
+        if (packed && log2_size <= 10)
+            hipLaunchKernelGGL(k_encode<uint32_t>, dim3(eblocks), dim3(kBlock), hist_bytes, s, enc, seg, per_block);
+        else
+            hipLaunchKernelGGL(k_encode<uint64_t>, dim3(eblocks), dim3(kBlock), hist_bytes, s, enc, seg, per_block);
         if (counted)
             hipLaunchKernelGGL(k_run_scan, dim3(kBlock), dim3(kBlock), 0, s, run_sum, run_sum + (uint64_t)eblocks * radix,
                                eblocks);

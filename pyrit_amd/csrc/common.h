@@ -25,6 +25,18 @@ __device__ __forceinline__ uint64_t local_key(uint32_t x, uint32_t y, uint32_t z
     return (brick << 6) | ((x & 3) + 4 * (y & 3) + 16 * (z & 3));
 }
 
+// The same for grids of edge up to 2^10, whose keys fit 30 bits: 32-bit
+// operations only.
+__device__ __forceinline__ uint32_t spread3_8(uint32_t v) {  // v < 2^8
+    uint32_t x = (v | (v << 8)) & 0x00F00Fu;
+    x = (x | (x << 4)) & 0x0C30C3u;
+    return (x | (x << 2)) & 0x249249u;
+}
+__device__ __forceinline__ uint32_t local_key32(uint32_t x, uint32_t y, uint32_t z) {
+    const uint32_t brick = spread3_8(x >> 2) | (spread3_8(y >> 2) << 1) | (spread3_8(z >> 2) << 2);
+    return (brick << 6) | (x & 3) | ((y & 3) << 2) | ((z & 3) << 4);
+}
+
 __host__ __device__ __forceinline__ uint32_t local_bits(uint32_t log2_size) { return 3 * (log2_size - 2) + 6; }
 
 // 64-bit finalizer used to place masks and node tuples in the hash tables; the
