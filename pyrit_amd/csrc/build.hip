@@ -1546,37 +1546,39 @@ __device__ __forceinline__ uint64_t level_insert_one(const LevelArgs& a, uint32_
 
 // node_heads/node_build/node_insert/node_owner (gbuild.zig:475-550) in one
 // pass: parents are numbered by a tile scan of the head flags, each head
-// gathers its <= 8 children, and the tuple is inserted into the level's hash
+// gathers its <= 8 children, and the tuple is inserted into the level's hash.
+// The heads of a tile (one element in eight where the grid is solid) are listed
+// in LDS first, so that every lane gathers one instead of one lane in eight
+// (bottom level of the 1024^3 grid 292 -> 159 us, of a 2048^3 surface 61 -> 28).
 __global__ void __launch_bounds__(kBlock) k_level_build(ScanCtx sc, LevelArgs a) {
     __shared__ uint32_t s_tile, s_wave[4];
     __shared__ uint64_t s_b;
+    __shared__ uint16_t s_head[kScanTile];
     const uint32_t n = min(sc.counters[C_NCH + a.lv], a.ch_cap);
     const uint32_t ntiles = (n + kScanTile - 1) / kScanTile;
     for (;;) {
         const uint32_t tile = next_tile(sc, &s_tile);
         if (tile >= ntiles) break;
         uint32_t f[kScanItems], e[kScanItems];
-        uint64_t k[kScanItems];
+        const uint64_t base = (uint64_t)tile * kScanTile;
 #pragma unroll
         for (int i = 0; i < kScanItems; i++) {
             uint64_t idx = scan_index(tile, i);
             f[i] = 0;
-            if (idx < n) {
-                k[i] = a.ch.key[idx];
-                f[i] = level_head(a, idx, k[i]);
-            }
+            if (idx < n) f[i] = level_head(a, idx, a.ch.key[idx]);
         }
         uint32_t total = tile_scan<kScanItems>(f, e, s_wave);
-        uint64_t pre = tile_prefix(sc, tile, total, &s_b);
 #pragma unroll
-        for (int i = 0; i < kScanItems; i++) {
-            if (!f[i]) continue;
-            const uint64_t idx = scan_index(tile, i);
-            if (pre + e[i] >= a.par_cap) {  // only after a failed look-back
-                atomicOr(&sc.counters[C_ERR], 16u);
-                continue;
-            }
-            level_tuple(a, idx, n, k[i], (uint32_t)(pre + e[i]));
+        for (int i = 0; i < kScanItems; i++)
+            if (f[i]) s_head[e[i]] = (uint16_t)(scan_index(tile, i) - base);
+        uint64_t pre = tile_prefix(sc, tile, total, &s_b);  // (its barrier completes the list)
+        if (pre + total > a.par_cap) {  // only after a failed look-back
+            if (threadIdx.x == 0) atomicOr(&sc.counters[C_ERR], 16u);
+            continue;
+        }
+        for (uint32_t h = threadIdx.x; h < total; h += kBlock) {
+            const uint64_t idx = base + s_head[h];
+            level_tuple(a, idx, n, a.ch.key[idx], (uint32_t)(pre + h));
         }
         if (tile == ntiles - 1 && threadIdx.x == 0) sc.counters[C_NCH + a.lv + 1] = (uint32_t)(pre + total);
     }
