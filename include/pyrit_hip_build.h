@@ -60,7 +60,10 @@ typedef struct PyrhipChunkBatch {
     uint64_t chunk_log2;
 } PyrhipChunkBatch;
 
-/* Tuning of one build. Every setting gives the same output; they trade
+/* Tuning of one build. A single build whose settings all have their default
+ * values takes a table of one word per voxel instead of the sort when its grid
+ * is small (edge 2^6, or 2^7 with a record per 16 voxels). Every setting gives
+ * the same output; they trade
  * passes, tile sizes (the work of one 256-thread block), LDS footprint,
  * occupancy and hash probe lengths. A field left 0 takes the value installed
  * for the build's workload class by pyrhip_autotune / pyrhip_tuning_set, else
@@ -83,8 +86,10 @@ typedef struct PyrhipBuildTuning {
                                offsets from per-tile digit counts the encode step writes (later passes use the
                                decoupled look-back); 2: decoupled look-back in every pass */
     uint32_t levels;        /* node levels: 2 one workgroup builds every level in one launch, 1 four launches
-                               per level over the whole GPU, 0 (default): 2 when the build holds at most
-                               32768 bricks (its brick bound), else 1; the output is the same */
+                               per level over the whole GPU, 0 (default): the levels whose cells are few are
+                               laid out by cell (two launches each, the last ones one launch), and a build of
+                               at most 32768 bricks (its brick bound) in a large grid takes 2, the lower
+                               levels of other builds 1; the output is the same */
 } PyrhipBuildTuning;
 
 /* gpu_build.build (src/gpu_build.zig:94-96): DAG of n_old sorted unique
