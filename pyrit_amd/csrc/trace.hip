@@ -493,8 +493,10 @@ __device__ PyrHit trace_scene(const PyrScene& s, const float o[3], const float d
     // reciprocal directions. Subtraction and multiplication round monotonically,
     // so the range of the corners' products holds every ray's own product, and
     // an instance that fails the test fails it for each of the rays. Those that
-    // pass are visited in their order. (Undefined and infinite numbers give no
-    // range: then every instance is a candidate.)
+    // pass are visited in their order. (Undefined and infinite numbers of an
+    // origin or direction give no range: then every instance is a candidate. An
+    // undefined limit of a ray is none, as in visit(): the larger and the smaller
+    // of it and a number are the number.)
     Range ro[3], ri[3];
     bool finite = true;
 #pragma unroll
@@ -504,10 +506,10 @@ __device__ PyrHit trace_scene(const PyrScene& s, const float o[3], const float d
         ri[a] = wave_range(inv[a]);
     }
     const bool ranges = __ballot(!finite) == 0;
-    const float near = -wave_max(-tmin);
+    const float near = -wave_max(tmin == tmin ? -tmin : __builtin_inff());
     for (uint32_t base = 0; base < s.instance_count; base += kWave) {
         const uint32_t j = base + lane_id();
-        const float far = wave_max(best);
+        const float far = wave_max(best == best ? best : __builtin_inff());
         bool candidate = j < s.instance_count;
         if (candidate) {
             const PYR_CONSTANT PyrInstanceData& in = inst[j];
