@@ -18,6 +18,7 @@
 // kernels (k_dense_spread lays a general level out by cell).
 #pragma once
 #include "common.h"
+#include "dense_walk.h"
 
 namespace pyr {
 
@@ -71,14 +72,13 @@ __global__ void __launch_bounds__(kBlock) k_dense_scatter(DenseArgs a) {
     const uint32_t n = a.n_old + a.n_new, stride = gridDim.x * kBlock;
     const int32_t edge = 1 << a.log2_size;
     const uint64_t slots = (uint64_t)a.bricks * 64;
-    for (uint32_t g0 = blockIdx.x * kBlock + threadIdx.x; g0 < n; g0 += stride * kDenseUnroll) {
+    for (DenseWalk w(blockIdx.x * kBlock + threadIdx.x, stride, n); w.more(); w.next(kDenseUnroll)) {
         uint64_t key[kDenseUnroll];
 #pragma unroll
         for (int u = 0; u < kDenseUnroll; u++) {
-            const uint64_t g = (uint64_t)g0 + (uint64_t)u * stride;
             key[u] = ~0ull;
-            if (g >= n) continue;
-            const uint32_t i = n - 1 - (uint32_t)g;
+            if (!w.has(u)) continue;
+            const uint32_t i = w.record(u);
             if (i < a.n_old) {
                 key[u] = a.old_keys[i];
             } else {
@@ -90,7 +90,7 @@ __global__ void __launch_bounds__(kBlock) k_dense_scatter(DenseArgs a) {
 #pragma unroll
         for (int u = 0; u < kDenseUnroll; u++) {
             if (key[u] >= slots) continue;  // out of range, or past the last record
-            const uint32_t i = n - 1 - (g0 + (uint32_t)u * stride);
+            const uint32_t i = w.record(u);
             if (a.table[key[u]] <= i) atomicMax(&a.table[key[u]], i + 1);
         }
     }
@@ -277,7 +277,7 @@ __global__ void __launch_bounds__(kBlock) k_dense_spread(const uint32_t* counter
                                                           const uint32_t* count, DenseLevel to, uint32_t cells,
                                                           uint32_t* err) {
     const uint32_t n = min(counters[count_slot], cap), stride = gridDim.x * kBlock;
-    for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += stride) {
+    for (uint64_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += stride) {
         const uint64_t c = key[i];
         if (c >= cells) {  // only after a failed look-back
             atomicOr(err, 16u);
