@@ -2378,6 +2378,12 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
     const bool packed = key_bits <= 32 && rb == 8 && tun.pair_layout != 1;
     const uint32_t radix = 1u << rb;
     const uint64_t k = enc.chunk_count ? enc.chunk_count : 1;
+    // record tiles: a single build has exactly ceil(n / tile); a batch's are
+    // counted on the device, at most one partial tile more per chunk
+    const uint32_t sort_tile = kBlock * sort_items;
+    const uint64_t sort_tiles = ((uint64_t)nmax + sort_tile - 1) / sort_tile + (enc.chunk_count ? enc.chunk_count : 0);
+    if (sort_tiles * sort_tile >= 0xFFFFFFFFull)
+        return fail(PYR_ERROR_INVALID_ARGUMENT, "too many voxels and chunks for one build");
     if (!enc.chunk_count && !gb && !fixed && dense_build(tun, log2_size, n)) return run_dense(enc, log2_size, s, out);
 
     // upper bounds (gpu_build.zig:142-154, 291-300)
@@ -2435,12 +2441,6 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
     const uint64_t hist_words = (uint64_t)passes * segs * radix;
     uint32_t* hist;
     A.want(hist, hist_words * 2);
-    const uint32_t sort_tile = kBlock * sort_items;
-    // record tiles: a single build has exactly ceil(n / tile); a batch's are
-    // counted on the device, at most one partial tile more per chunk
-    const uint64_t sort_tiles = (nmax + sort_tile - 1) / sort_tile + (enc.chunk_count ? enc.chunk_count : 0);
-    if (sort_tiles * sort_tile >= 0xFFFFFFFFull)
-        return fail(PYR_ERROR_INVALID_ARGUMENT, "too many voxels and chunks for one build");
     Segs seg{};
     seg.single = enc.chunk_count == 0;
     seg.count = segs;

@@ -1,6 +1,8 @@
 """The dense build at record counts near 2^32: the rounds of its scatter end
 and take every record once (pyrit_amd/csrc/dense_walk.h, compiled for the host
-with g++; no GPU)."""
+with g++), and counts that no build takes are refused before any device work,
+on small grids as on large ones (no GPU)."""
+import ctypes as C
 import os
 import subprocess
 
@@ -33,3 +35,16 @@ def test_rounds_end(walk, n):
         assert taken == want and regular
         if taken:
             assert first == n - 1 - thread and last == (n - 1 - thread) % threads
+
+
+@pytest.mark.parametrize("log2", [3, 5, 6, 7, 8, 12])
+def test_counts_refused(log2):
+    from pyrit_amd import abi, lib
+
+    L = lib()
+    out, t = abi.PyrhipBuilt(), abi.PyrhipBuildTuning()
+    # (the addresses are never used: the count is refused first)
+    for n_old, n_new in ((0, 2 ** 32 - 2), (0, 2 ** 32 - 3000), (2 ** 31, 2 ** 31 - 2)):
+        code = L.pyrhip_build(log2, 4096 if n_old else 0, 4096 if n_old else 0, n_old, 4096, n_new, C.byref(t), None,
+                              C.byref(out))
+        assert code == abi.PYR_ERROR_INVALID_ARGUMENT, (n_old, n_new, code)
