@@ -62,8 +62,8 @@ typedef struct PyrhipChunkBatch {
 
 /* Tuning of one build. A single build whose settings all have their default
  * values takes a table of one word per voxel instead of the sort when its grid
- * is small (edge 2^6, or 2^7 with a record per 16 voxels). Every setting gives
- * the same output; they trade
+ * is small: edge up to 2^5, 2^6 with at most 2^26 records, 2^7 with a record per
+ * 16 voxels and at most 2^24. Every setting gives the same output; they trade
  * passes, tile sizes (the work of one 256-thread block), LDS footprint,
  * occupancy and hash probe lengths. A field left 0 takes the value installed
  * for the build's workload class by pyrhip_autotune / pyrhip_tuning_set, else

@@ -2135,8 +2135,17 @@ struct FixedMemory {
 // per voxel of the grid, at most 1 MiB (edge 2^6) or 64 bytes per record, which
 // is what the sorted build's buffers take. A call that names a setting other
 // than the defaults gets the kernels that the setting is about.
+// Neighbouring records of one voxel wait for each other's atomics, so a grid
+// with very many records a voxel gains or loses by their order (us, dense and
+// sorted): 1.6e7 records of a 2^7 grid in voxel order 643 and 363, random 466 and
+// 425, sweep after sweep over the grid 187 and 363, most of them in few voxels
+// 906 and 2601; 1e8 in voxel order 4791 and 1555. The lines keep that loss
+// bounded: 2^24 records of a 2^7 grid; 2^26 of a 2^6 grid, whose orders come out
+// alike there (shuffled within 4096: 6.4e7 records 1740 and 1694, 1e8 2998 and
+// 2556); none below, where the table is faster at every count measured.
 bool dense_build(const PyrhipBuildTuning& tun, uint32_t log2_size, uint64_t n) {
     if (n == 0 || log2_size > 7 || !default_tuning(tun)) return false;
+    if (log2_size >= 6 && n > 1ull << (log2_size == 7 ? 24 : 26)) return false;
     const uint64_t slots = 1ull << (3 * log2_size);
     return slots <= (1ull << 18) || slots <= 16 * n;
 }

@@ -49,6 +49,26 @@ def test_rule_edge(hip_device):
     assert_same_build(_build(5, pts, True, sort_items=20), ref, 5)
 
 
+def test_many_records_are_sorted(hip_device):
+    """The last record count of a 2^7 grid that the table takes, and one more
+    (a record outside the grid): the same voxels, by the table and sorted."""
+    from pyrit_amd import abi
+
+    count = 1 << 24
+    pts = np.zeros(count + 1, abi.VOXEL)
+    rng = np.random.default_rng(24)
+    i = np.arange(count) // 8  # in voxel order, eight records each
+    pts["x"][1:], pts["y"][1:], pts["z"][1:] = i % 128, i // 128 % 128, i // 16384
+    pts["attribute"][1:] = rng.integers(0, 5, count)
+    pts["x"][0], pts["attribute"][0] = -1, 7
+    a, b = _build(7, pts[1:], True), _build(7, pts, False)
+    # the last record of a voxel wins; attribute 0 removes it
+    assert a.voxel_count == np.count_nonzero(pts["attribute"][8::8])
+    for what in ("nodes", "leaves", "keys", "attrs"):
+        assert np.array_equal(getattr(a, what)(), getattr(b, what)()), what
+    assert a.root == b.root
+
+
 @pytest.mark.parametrize("log2,edits", [(3, 1), (5, 700), (6, 4096), (7, 311)])
 def test_edits(hip_device, log2, edits):
     from pyrit_amd import gpu as g
