@@ -2095,6 +2095,13 @@ void launch_unique_bricks(hipStream_t s, uint32_t items, uint32_t sort_tile, uin
 // cells (and without): 2^9 terrain 2152, 2119, 2063, 2024 (2260) us, 2^11
 // surface 1500, 1428, 1378, 1473 (1562), 48 chunks 1609, 1577, 1503, 1587 (1648).
 constexpr uint64_t kDenseCells = 1ull << 18;
+// Bricks from which dense levels above lv0 are faster than k_levels_small, for
+// a build that knows its bricks: one workgroup pays by the brick, the general
+// levels below lv0 by the level (us, one workgroup and dense): no general level,
+// 500 bricks 245 and 255, 2000 264 and 257; one, 2000 231 and 236, 4000 252 and
+// 242; two, 2560 219 and 245, 3200 290 and 276; three, 4000 316 and 335, 8000 380
+// and 342; six, 2000 283 and 330, 4000 368 and 403, 8000 473 and 436.
+constexpr uint64_t dense_bricks(uint32_t lv0) { return std::min<uint64_t>(4096, 1024ull * (lv0 - 1)) + 1; }
 
 // A chunk-batch build captured into a HIP graph (pyrhip_graph_*): every
 // buffer is allocated once for the largest batch, the kernels take their
@@ -2505,13 +2512,13 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
     // the levels from lv0 up are dense (dense.h) when their cells are few (16
     // bytes each: at most 8 per record beyond those of the last kernel): all
     // of them, or those above the levels of a build with more bricks than one
-    // workgroup takes
+    // workgroup takes; a build that reads its brick count back and finds few
+    // leaves its levels to that one workgroup after all (dense_bricks)
     uint32_t lv0 = 2;
     const uint64_t cells_max = std::min<uint64_t>(kDenseCells, std::max<uint64_t>(kDenseTop, nmax / 2));
     while (lv0 < log2_size && (k << (3 * (log2_size - lv0))) > cells_max) lv0++;
     const uint64_t dense_cells = k << (3 * (log2_size - lv0));
-    const bool dense_levels = tun.levels == 0 && !fixed && k <= kDenseTop && (lv0 == 2 || nb > kLevelsSmallBricks);
-    if (!dense_levels) lv0 = log2_size;
+    bool dense_levels = tun.levels == 0 && !fixed && k <= kDenseTop && (lv0 == 2 || nb > kLevelsSmallBricks);
     DenseLevels dense(lv0, dense_levels ? dense_cells : 0, nmax);
     DenseLevel dense_from{};  // the cells of level lv0
     uint32_t* dense_zero = nullptr;
@@ -2710,6 +2717,7 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
             return fail(PYR_ERROR_CUDA, "build: %s", hipGetErrorString(be));
         }
         lz = level_sizes(std::min<uint64_t>(bricks, nb));  // (a failed unique step may report anything)
+        if (lz.nb < dense_bricks(lv0)) dense_levels = false;
         if (!alloc_levels()) {
             A.release();
             free_outputs();
@@ -2717,6 +2725,7 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
             return fail(PYR_ERROR_OUT_OF_MEMORY, "device memory for a build of %u voxels", n);
         }
     }
+    if (!dense_levels) lv0 = log2_size;
     // 4. leaves
     const uint32_t brick_grid = grid_for(lz.nb, kScanTile, 2048);
     hipLaunchKernelGGL(k_hash_clear, dim3(grid_for(lz.cap, 1024, 2048)), dim3(kBlock), 0, s, counters, (uint32_t)C_B,

@@ -166,3 +166,41 @@ def test_upper_levels(hip_device, log2, n):
     one["x"] = one["y"] = one["z"] = (1 << log2) - 1
     many = np.repeat(one, 70000)  # one voxel of many records in a large grid
     assert_same_build(g.build(log2, many), O.gb_build(log2, many), log2)
+
+
+def _patch(log2, bricks, per, seed):
+    """`per` random voxels in each of `bricks` bricks side by side"""
+    rng = np.random.default_rng(seed)
+    side = min(1 << (log2 - 2), int(np.ceil(np.sqrt(bricks))))
+    b = np.repeat(np.arange(bricks), per)
+    bit = np.argsort(rng.random((bricks, 64)), 1)[:, :per].ravel()
+    pts = np.zeros(len(b), O.VOXEL)
+    pts["x"] = b % side * 4 + (bit & 3)
+    pts["y"] = b // side // side * 4 + (bit >> 2 & 3)
+    pts["z"] = b // side % side * 4 + (bit >> 4)
+    pts["attribute"] = rng.integers(1, 1 << 20, len(b))
+    rng.shuffle(pts)
+    return pts
+
+
+@pytest.mark.parametrize("log2,bricks,repeat,small", [(9, 3072, 1, True), (9, 3073, 1, False), (13, 700, 4, True),
+                                                      (8, 2048, 3, True), (8, 2049, 3, False), (8, 1024, 20, True),
+                                                      (8, 1025, 20, False)])
+def test_levels_of_few_bricks(hip_device, log2, bricks, repeat, small):
+    """Builds of many records in few bricks of a large grid: the levels of one
+    workgroup up to the brick count where dense ones become faster (a build
+    that takes those holds the same memory as one asked to), and equal arrays."""
+    from pyrit_amd import gpu as g
+
+    pts = np.tile(_patch(log2, bricks, 32, bricks), repeat)
+    ref = O.gb_build(log2, pts)
+    held = {}
+    g.set_timing(True)
+    try:
+        for levels in (0, 2, 1):
+            assert_same_build(g.build(log2, pts, levels=levels), ref, log2)
+            held[levels] = g.last_build_times()["device_bytes"]
+    finally:
+        g.set_timing(False)
+    assert (held[0] == held[2]) == small, held
+    assert held[1] == held[2]
