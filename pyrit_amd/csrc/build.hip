@@ -2178,6 +2178,11 @@ struct DenseLevels {
         for (uint32_t i = 0; i < wides; i++) w += 2ull * wide[i].cap;
         return w;
     }
+    uint64_t bytes() const {  // of what want() takes
+        uint64_t b = 0;
+        for (uint32_t i = 0; i < wides; i++) b += 16ull * wide[i].parents;
+        return b;
+    }
     void want(Alloc& A) {
         for (uint32_t i = 0; i < wides; i++) {
             A.want(wide[i].cells.rep, wide[i].parents);
@@ -2436,14 +2441,27 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
         return z.cap * 12 + z.nb * (4 + 12 + 8) + z.np2 * (20 + (uint64_t)kNodeStride * 4 + 4) + z.words * 4;
     };
     LevelSizes lz = level_sizes(nb);
+    // the levels from lv0 up are dense (dense.h) when their cells are few (16
+    // bytes each: at most 8 per record beyond those of the last kernel): all
+    // of them, or those above the levels of a build with more bricks than one
+    // workgroup takes; a build that reads its brick count back and finds few
+    // leaves its levels to that one workgroup after all (dense_bricks)
+    uint32_t lv0 = 2;
+    const uint64_t cells_max = std::min<uint64_t>(kDenseCells, std::max<uint64_t>(kDenseTop, nmax / 2));
+    while (lv0 < log2_size && (k << (3 * (log2_size - lv0))) > cells_max) lv0++;
+    const uint64_t dense_cells = k << (3 * (log2_size - lv0));
+    bool dense_levels = tun.levels == 0 && !fixed && k <= kDenseTop && (lv0 == 2 || nb > kLevelsSmallBricks);
+    DenseLevels dense(lv0, dense_levels ? dense_cells : 0, nmax);
+    const uint64_t dense_words = (dense_cells + dense.zero_words() + 3) & ~3ull;
+    const uint64_t dense_bytes = dense_levels ? dense_cells * 8 + dense_words * 4 + dense.bytes() : 0;
     // when the bounds would hold more than 8 bytes per record plus 1 MiB for
-    // the brick-sized buffers (sparse inputs with about one brick per record,
-    // batches whose chunk cells far exceed their bricks) the build reads the
-    // brick count back once after the unique step and sizes them exactly, so
-    // a build never holds more than that beyond its real need; smaller
-    // builds skip the read-back; graph captures and the static scratch keep
-    // the bounds
-    const bool exact_levels = !gb && !fixed && level_bytes(lz) > 8ull * nmax + (1ull << 20);
+    // the brick-sized buffers and the dense levels (sparse inputs with about
+    // one brick per record, batches whose chunk cells far exceed their bricks)
+    // the build reads the brick count back once after the unique step and
+    // sizes the former exactly, so a build never holds more than that beyond
+    // its real need (dense levels alone hold less); smaller builds skip the
+    // read-back; graph captures and the static scratch keep the bounds
+    const bool exact_levels = !gb && !fixed && level_bytes(lz) + dense_bytes > 8ull * nmax + (1ull << 20);
 
     const auto host_t0 = std::chrono::steady_clock::now();
     Alloc A{{}, s};
@@ -2509,20 +2527,8 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
     uint64_t* table = nullptr;
     uint32_t* owner = nullptr;
     uint32_t* slot = nullptr;
-    // the levels from lv0 up are dense (dense.h) when their cells are few (16
-    // bytes each: at most 8 per record beyond those of the last kernel): all
-    // of them, or those above the levels of a build with more bricks than one
-    // workgroup takes; a build that reads its brick count back and finds few
-    // leaves its levels to that one workgroup after all (dense_bricks)
-    uint32_t lv0 = 2;
-    const uint64_t cells_max = std::min<uint64_t>(kDenseCells, std::max<uint64_t>(kDenseTop, nmax / 2));
-    while (lv0 < log2_size && (k << (3 * (log2_size - lv0))) > cells_max) lv0++;
-    const uint64_t dense_cells = k << (3 * (log2_size - lv0));
-    bool dense_levels = tun.levels == 0 && !fixed && k <= kDenseTop && (lv0 == 2 || nb > kLevelsSmallBricks);
-    DenseLevels dense(lv0, dense_levels ? dense_cells : 0, nmax);
     DenseLevel dense_from{};  // the cells of level lv0
     uint32_t* dense_zero = nullptr;
-    const uint64_t dense_words = (dense_cells + dense.zero_words() + 3) & ~3ull;
     LevelArrays set[2];
     uint32_t* node_tmp = nullptr;
     uint32_t* node_len = nullptr;

@@ -204,3 +204,23 @@ def test_levels_of_few_bricks(hip_device, log2, bricks, repeat, small):
         g.set_timing(False)
     assert (held[0] == held[2]) == small, held
     assert held[1] == held[2]
+
+
+def test_memory_of_dense_levels(hip_device):
+    """2.1e6 records in 20000 bricks of a 2^8 grid: the brick-sized buffers for
+    the most bricks there can be hold 16.2 MB, within 8 bytes a record plus
+    1 MiB (17.8 MB), but 20.5 MB with the dense levels: such a build counts its
+    bricks and holds less than one without dense levels."""
+    from pyrit_amd import gpu as g
+
+    pts = np.tile(_patch(8, 20000, 35, 1), 3)
+    ref = O.gb_build(8, pts)
+    held = []
+    g.set_timing(True)
+    try:
+        for levels in (0, 1):
+            assert_same_build(g.build(8, pts, levels=levels), ref, 8)
+            held.append(g.last_build_times()["device_bytes"])
+    finally:
+        g.set_timing(False)
+    assert held[0] < held[1], held
