@@ -1806,7 +1806,8 @@ __global__ void __launch_bounds__(kLevelsBlock) k_levels_small(uint32_t* counter
 // roots of the top level and the empty geometry (gbuild.zig:607-624)
 __global__ void __launch_bounds__(kBlock) k_finalize(uint32_t* counters, uint32_t top, LevelArrays par,
                                                       uint32_t* roots, uint32_t* nodes_out, uint32_t par_cap,
-                                                      uint32_t chunk_count, uint64_t word_cap, uint32_t* host) {
+                                                      uint32_t chunk_count, uint64_t word_cap, uint32_t* host,
+                                                      uint32_t host_roots) {
     const uint32_t np = min(counters[C_NCH + top], par_cap);
     const uint32_t cur = counters[C_CUR + top];
     if (roots) {
@@ -1828,11 +1829,12 @@ __global__ void __launch_bounds__(kBlock) k_finalize(uint32_t* counters, uint32_
         counters[C_ROOT] = root;
         counters[C_WORDS] = words;
     }
-    // into the caller's pinned words: counters, roots, first voxels
+    // into the caller's pinned words: counters, and the roots and first voxels
+    // of `host_roots` chunks
     __syncthreads();
     if (!host) return;
     for (uint32_t i = threadIdx.x; i < C_TILE; i += kBlock) host[i] = counters[i];
-    for (uint32_t i = threadIdx.x; i < 2 * chunk_count; i += kBlock) host[C_TILE + i] = roots[i];
+    for (uint32_t i = threadIdx.x; i < 2 * host_roots; i += kBlock) host[C_TILE + i] = roots[i];
 }
 
 __device__ __forceinline__ uint32_t compact3(uint64_t v) {
@@ -2103,10 +2105,18 @@ constexpr uint64_t kDenseCells = 1ull << 18;
 // and 342; six, 2000 283 and 330, 4000 368 and 403, 8000 473 and 436.
 constexpr uint64_t dense_bricks(uint32_t lv0) { return std::min<uint64_t>(4096, 1024ull * (lv0 - 1)) + 1; }
 
+// Roots and first voxels of at most this many chunks are written into pinned
+// words by the build's last kernel; a longer list is copied, as one workgroup's
+// writes over the bus are slower than that (us, written and copied: 6000 chunks
+// of edge 2^3 985 and 1030, 10000 1152 and 1190, 20000 2013 and 2005, 100000 9065
+// and 8780).
+constexpr uint32_t kHostRoots = 16384;
+static_assert(kHostRoots >= kDenseTop, "k_dense_top writes the roots of every build it ends");
+
 // A chunk-batch build captured into a HIP graph (pyrhip_graph_*): every
 // buffer is allocated once for the largest batch, the kernels take their
 // sizes from the device arrays (offsets, counters), and a replay ends with
-// the counters, roots and first voxels copied into pinned host memory.
+// the counters, roots and first voxels in pinned host memory.
 struct GraphBuild {
     std::vector<void*> scratch;
     uint64_t* kb[2] = {nullptr, nullptr};
@@ -2588,7 +2598,8 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
     seg.tiles = counters + C_TILES;
     // the read-back: pinned words that the last kernel writes
     // (a build without allocation copies them into `local` instead)
-    HostWords back(gb || fixed ? 0 : C_TILE + 2ull * enc.chunk_count);
+    const uint32_t host_roots = enc.chunk_count <= kHostRoots ? enc.chunk_count : 0;
+    HostWords back(gb || fixed ? 0 : C_TILE + 2ull * host_roots);
     uint32_t local[C_TILE];
     out_ok &= gb || fixed || back.p;
     auto free_outputs = [&]() {
@@ -2816,7 +2827,8 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
                      gb ? gb->host : back.p);
     } else {
         hipLaunchKernelGGL(k_finalize, dim3(1), dim3(kBlock), 0, s, counters, log2_size, set[ch], roots_dev, nodes_out,
-                           (uint32_t)std::min(set_cap[ch], lz.np2), enc.chunk_count, lz.words, gb ? gb->host : back.p);
+                           (uint32_t)std::min(set_cap[ch], lz.np2), enc.chunk_count, lz.words, gb ? gb->host : back.p,
+                           host_roots);
     }
     tm.mark();
 
@@ -2824,6 +2836,15 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
     const uint32_t* const c = gb ? gb->host : fixed ? local : back.p;
     hipError_t e = hipSuccess;
     if (fixed) e = hipMemcpyAsync(local, counters, sizeof(local), hipMemcpyDeviceToHost, s);
+    if (enc.chunk_count > host_roots) {
+        if (gb) {
+            roots_host = gb->host + C_TILE;
+            first_host = roots_host + enc.chunk_count;
+        }
+        e = hipMemcpyAsync(roots_host, roots_dev, enc.chunk_count * 4ull, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(first_host, first_dev, enc.chunk_count * 4ull, hipMemcpyDeviceToHost, s);
+    }
     if (gb) {
         hipGraph_t graph = nullptr;
         const hipError_t ce = hipStreamEndCapture(s, &graph);
@@ -2854,7 +2875,7 @@ PyrResult run_build(const EncodeArgs& enc_in, uint32_t log2_size, const PyrhipBu
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     const auto host_t3 = std::chrono::steady_clock::now();
     if (e == hipSuccess) e = hipGetLastError();
-    if (enc.chunk_count && e == hipSuccess) {
+    if (host_roots && e == hipSuccess) {
         memcpy(roots_host, c + C_TILE, enc.chunk_count * 4ull);
         memcpy(first_host, c + C_TILE + enc.chunk_count, enc.chunk_count * 4ull);
     }

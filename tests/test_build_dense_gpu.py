@@ -224,3 +224,28 @@ def test_memory_of_dense_levels(hip_device):
     finally:
         g.set_timing(False)
     assert held[0] < held[1], held
+
+
+@pytest.mark.parametrize("count", [16384, 16385])
+def test_many_chunks(hip_device, count):
+    """The most chunks whose roots the last kernel writes to the host, and one
+    more (they are copied): as a batch, and replayed as a graph with fewer."""
+    from pyrit_amd import gpu as g
+
+    rng = np.random.default_rng(count)
+    sizes = rng.integers(0, 5, count)
+    offs = np.concatenate([[0], np.cumsum(sizes)]).astype(np.uint32)
+    vox = random_points(int(offs[-1]), 3, 1, dup_frac=0.0)
+    vox["attribute"][::50] = 0
+    ref, rroots, rfirst = O.gb_build_chunks(3, vox, offs)
+    graph = g.BuildGraph(3, count, len(vox))
+    try:
+        for few in (count, 100, count):
+            cut = offs.copy()
+            cut[few:] = offs[few]
+            want, wroots, wfirst = (ref, rroots, rfirst) if few == count else O.gb_build_chunks(3, vox[:cut[-1]], cut)
+            for b, roots, first in (graph.launch(vox[:cut[-1]], cut), g.build_chunks(3, vox[:cut[-1]], cut)):
+                assert_same_build(b, want, 3)
+                assert np.array_equal(roots, wroots) and np.array_equal(first, wfirst)
+    finally:
+        graph.destroy()
