@@ -435,6 +435,51 @@ def _decode(m):
     return tuple(out)
 
 
+@pytest.mark.parametrize("finish", [0, 1, 2])
+def test_small_grids_on_every_build(hip_device, finish):
+    """Small grids take the table build by default (reported as finish 0); the
+    sorted one with either finish gives the same arrays for the inputs that
+    its leaf hash, its empty geometry and its edits are to be tested with."""
+    g = _gpu()
+
+    def build(log2, pts, old=None):
+        g.set_timing(True)
+        try:
+            b = g.build(log2, pts, old=old, finish=finish)
+            assert g.last_build_times()["finish"] == finish
+        finally:
+            g.set_timing(False)
+        return b
+
+    # leaf masks of one wave that differ in the high dword only, and in the low one only
+    for flip in (False, True):
+        pts = []
+        for m in range(64):
+            bx, by, bz = _decode(m)
+            bits = [31] if m == 0 else [31] + list(range(32, 64))
+            for bit in bits:
+                bit = 63 - bit if flip else bit
+                pts.append((bx * 4 + (bit & 3), by * 4 + ((bit >> 2) & 3), bz * 4 + (bit >> 4), 5 + m))
+        pts = np.array(pts, O.VOXEL)
+        ref = O.gb_build(5, pts)
+        assert len(ref["leaves"]) == 2
+        assert_same_build(build(5, pts), ref, 5)
+    pts = grid_to_points(scene_grid(64))
+    np.random.default_rng(3).shuffle(pts)
+    ref = O.gb_build(6, pts)
+    b = build(6, pts)
+    assert_same_build(b, ref, 6)
+    ed = random_points(3000, 6, 17, dup_frac=0.2, delete_frac=0.4, out_frac=0.05)
+    assert_same_build(build(6, ed, old=b), O.gb_build(6, ed, ref["keys"], ref["attrs"]), 6)
+    gone = pts.copy()
+    gone["attribute"] = 0
+    for log2, none, old in ((5, np.array([(1, 1, 1, 0), (99, 0, 0, 3), (-1, 2, 2, 4)], O.VOXEL), None), (6, gone, b)):
+        e = build(log2, none, old)
+        assert e.voxel_count == 0 and e.leaf_count == 0 and e.nodes().tolist() == [0, 0] and e.root == 0
+    one = np.array([(5, 6, 7, 42)], O.VOXEL)
+    assert_same_build(build(4, one), O.gb_build(4, one), 4)
+
+
 def test_edit_equals_rebuild(hip_device):
     # cpu_test.zig:809-850 on the GPU path
     print("case: edit = rebuild", flush=True)
