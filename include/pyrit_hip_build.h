@@ -87,9 +87,10 @@ typedef struct PyrhipBuildTuning {
                                decoupled look-back); 2: decoupled look-back in every pass */
     uint32_t levels;        /* node levels: 2 one workgroup builds every level in one launch, 1 four launches
                                per level over the whole GPU, 0 (default): the levels whose cells are few are
-                               laid out by cell (two launches each, the last ones one launch), and a build of
-                               at most 32768 bricks (its brick bound) in a large grid takes 2, the lower
-                               levels of other builds 1; the output is the same */
+                               laid out by cell (two launches each, the last ones one launch), the levels
+                               below them 1; a build of at most 32768 bricks (its brick bound) in a large
+                               grid, or of at most a few thousand where it counts them, takes 2; the output
+                               is the same */
 } PyrhipBuildTuning;
 
 /* gpu_build.build (src/gpu_build.zig:94-96): DAG of n_old sorted unique
@@ -193,7 +194,8 @@ typedef struct PyrhipTuneReport {
 PYR_API PyrResult pyrhip_autotune(uint32_t log2_size, uint64_t voxels, uint32_t n, const PyrhipChunkBatch* batch,
                                   uint32_t repeats, void* stream, PyrhipTuneReport* out);
 /* installs (tuning != NULL) or removes the setting of a class, e.g. one saved
- * from an earlier autotune run */
+ * from an earlier autotune run. Any value other than a default, of any field,
+ * keeps the small grids of that class on the sorted build. */
 PYR_API PyrResult pyrhip_tuning_set(uint32_t log2_size, uint32_t n, uint32_t chunk_count,
                                     const PyrhipBuildTuning* tuning);
 /* the setting a build of this class uses when its tuning fields are 0 */
@@ -234,7 +236,8 @@ typedef struct PyrhipBuildTimes {
      * waiting for the final read-back */
     float host_alloc_ms, host_enqueue_ms, host_wait_ms;
     uint32_t status_bytes; /* bytes per sort look-back word: 4 or 8 */
-    uint32_t finish;       /* 2: partial sort + bucket tables, 1: full sort + unique scan */
+    uint32_t finish;       /* 2: partial sort + bucket tables, 1: full sort + unique scan, 0: a table of one
+                              word per voxel instead of the sort (then the sort's fields are 0 too) */
     uint64_t device_bytes; /* device memory the build requested, scratch and outputs (all held at once:
                               the peak) */
 } PyrhipBuildTimes;

@@ -285,8 +285,8 @@ __device__ __forceinline__ void emit_record(const EncodeArgs& a, uint32_t* s_his
 
 // K: 32-bit keys for packed records of grids up to 2^10, 64 bits otherwise: the
 // 64-bit spreading of the coordinates was most of the kernel's vector work
-// (1024^3 grid, 5.1e8 records: 2.87 -> 2.38 ms, 5.1 TB/s; the copy probe reaches
-// 5.5).
+// (1024^3 grid, 5.1e8 records, kernel time: 2.84 -> 2.38 ms, 5.1 TB/s; the copy
+// probe reaches 5.5).
 template <typename K>
 __global__ void __launch_bounds__(kBlock) k_encode(EncodeArgs a, Segs g, uint32_t tiles_per_block) {
     extern __shared__ uint32_t s_hist[];
@@ -1122,7 +1122,7 @@ __global__ void __launch_bounds__(kBlock) k_bucket_bounds(const uint32_t* counte
 // A wave owns consecutive bricks and keeps their masks and prefixes in its
 // lanes: no LDS round trip per brick in the write-out (14.4 -> 9.3 us of a
 // bucket's 55 on the 1024^3 grid; the wait for the predecessors' counts takes
-// back part of it: 3.13 -> 2.95 ms), and brick keys and masks leave as whole
+// back part of it: 3.22 -> 3.07 ms), and brick keys and masks leave as whole
 // rows instead of one lane at a time.
 template <bool PACKED>
 __global__ void __launch_bounds__(kBucketBlock, 4)
@@ -1278,7 +1278,7 @@ __global__ void __launch_bounds__(kBucketBlock, 4)
                 continue;
             }
             const uint32_t br0 = wave * kWaveBricks;
-            uint32_t here = lane;
+            uint32_t here = lane;  // (as above: no addresses kept across buckets)
             asm volatile("" : "+v"(here));
             if (mask) {
                 brick_key[pre_b + before_b] = (base_key >> 6) | (br0 + lane);
@@ -2159,7 +2159,9 @@ struct FixedMemory {
 // 906 and 2601; 1e8 in voxel order 4791 and 1555. The lines keep that loss
 // bounded: 2^24 records of a 2^7 grid; 2^26 of a 2^6 grid, whose orders come out
 // alike there (shuffled within 4096: 6.4e7 records 1740 and 1694, 1e8 2998 and
-// 2556); none below, where the table is faster at every count measured.
+// 2556); none below, where the table is faster at every count measured. Grids of
+// edge 2^8 gain nothing (terrain of 8.5e6 records 424 and 414, random 1e6 371 and
+// 357, 4e6 524 and 434, 1.7e7 1058 and 687): their table is 64 MB.
 bool dense_build(const PyrhipBuildTuning& tun, uint32_t log2_size, uint64_t n) {
     if (n == 0 || log2_size > 7 || !default_tuning(tun)) return false;
     if (log2_size >= 6 && n > 1ull << (log2_size == 7 ? 24 : 26)) return false;

@@ -34,13 +34,14 @@ constexpr uint32_t kMaxSteps = 65536;
 // either way, 16 take 325 us with the test and 330 without, 64 take 476 and
 // 533, 1000 take 802 and 2429.)
 constexpr uint32_t kCullInstances = 8;
-// A launch whose rays make fewer waves than this takes fewer rays per wave: a
+// The most waves that a launch is spread over by halving its rays per wave: a
 // chip with idle slots gains from waves that diverge less and whose boxes
-// are smaller, a full one loses by the repeated lanes. The chip holds 8192
-// waves. One DAG (or a few instances): 1000 diffuse rays 55 -> 36 us, 16000
-// 88 -> 73, 64000 84 -> 81; 8192 waves take 89 us for the 64000, 16384 take
-// 115. Instances: a 640x360 frame of 64 takes 468 us with full waves, 383 with
-// at least 8192, 340 with 16384, 354 with 32768; of 1000: 633, 500, 432, 557.
+// are smaller, a full one loses by the repeated lanes. (Rays that fill more than
+// half as many waves are not spread.) The chip holds 8192 waves. One DAG (or a
+// few instances): 1000 diffuse rays 55 -> 36 us, 16000 88 -> 73, 64000 84 -> 81;
+// with up to 8192 waves the 64000 take 89 us, with up to 16384 115. Instances: a
+// 640x360 frame of 64 takes 468 us with full waves, 383 with up to 8192, 340
+// with 16384, 354 with 32768; of 1000: 633, 500, 432, 557.
 constexpr uint32_t kRayWaves = 4096, kSceneWaves = 16384;
 constexpr uint32_t kNotMoved = 4;  // added to the entry axis of a walk that has not left its first cell
 constexpr uint32_t kHit = 32, kMiss = 64;  // values of a finished walk's scale
@@ -217,8 +218,10 @@ __device__ bool walk(const DagView& g, const float o[3], const float d[3], float
     stk[scale * kTraceBlock] = g.root;
     // The levels that every lane of the wave enters the same way, node words
     // through the scalar cache: neighbouring primary and shadow rays share
-    // most of the way down to their first cell (shadow rays of a 4096^3
-    // landscape 112 -> 105 us per 1920x1080 frame, primary rays 279 -> 277).
+    // most of the way down to their first cell (six poses over a 4096^3
+    // landscape: 3840x2160 primary rays 671 -> 664 us a frame, 1920x1080 shadow
+    // rays 182 -> 179, 1920x1080 primary rays 229 either way; 64 instances 459 ->
+    // 456).
     {
         const uint32_t u0 = first_lane32(q[0]), u1 = first_lane32(q[1]), u2 = first_lane32(q[2]), uo = first_lane32(oct);
         const uint32_t apart = oct == uo ? (q[0] ^ u0) | (q[1] ^ u1) | (q[2] ^ u2) : ~0u;
@@ -241,18 +244,19 @@ __device__ bool walk(const DagView& g, const float o[3], const float d[3], float
     uint32_t steps = 0, iter = 0;
     // One iteration looks a cell up and enters it if it is filled, or leaves
     // it along the ray and ascends to the highest coordinate bit that changed.
-    // The walk is bound by instruction issue (vector ALU busy 83 % of a primary
+    // The walk is bound by instruction issue (vector ALU busy 78 % of a primary
     // frame), the scalar unit's share included, which the masks of nested
     // branches and of flags kept across them load as much as the arithmetic
     // does the vector unit. So there are three branches in a row and no exits
     // from inside them: an empty cell's step is formed whole also when it ends
     // the walk, and the end of a walk is a value of `scale`, not a flag.
-    // 1920x1080 frames of a 4096^3 landscape against the form that converted
-    // and compared coordinates at every level entered and left: primary
-    // 336 -> 253 us, shadow 135 -> 101 us, 1e6 diffuse rays 267 -> 209 us.
-    // (Measured and left out: entering until a cell is empty before any lane
-    // leaves one, 328 us; two lookups per iteration, 250 us, but shadow rays
-    // 103; the child loaded for empty cells too to save a branch, 258 us.)
+    // 1920x1080 frames of a 4096^3 landscape, mean of six poses, against the
+    // form that converted and compared coordinates at every level entered and
+    // left: primary 306 -> 229 us, shadow 236 -> 179 us; 1e6 diffuse rays 271 ->
+    // 215 us. (Measured and left out: entering until a cell is empty before any
+    // lane leaves one, primary 1.30 times as long; two lookups per iteration, 0.99,
+    // but shadow rays 1.02; the child loaded for empty cells too to save a
+    // branch, 1.02.)
     do {
         uint32_t filled = 1;
         if (scale >= 2) {
@@ -322,7 +326,7 @@ __device__ bool walk(const DagView& g, const float o[3], const float d[3], float
             t = max_f32(t, tnext);
             axis = s2 ? 2u : (a1 ? 1u : 0u);
             if (bounded) {
-                asm volatile("");
+                asm volatile("");  // (opaque, so that this stays a block of its own: without it 229 -> 240 us)
                 steps += up + 1 - scale;
                 leave |= steps + top - up >= kMaxSteps;
             }
@@ -651,7 +655,7 @@ __device__ __forceinline__ void camera_ray(const PyrCamera& c, uint32_t x, uint3
     *tmax = c.far_plane > 0 ? c.far_plane * len : PYR_FLT_MAX;
 }
 
-// 8x16 pixel tiles per workgroup keep a wave's rays coherent
+// pixel tiles (16 x 4 a wave in large frames) keep a wave's rays coherent
 __global__ void __launch_bounds__(kTraceBlock) k_trace_camera(DagView g, PyrCamera cam, PyrHit* hits,
                                                                uint32_t flags, uint32_t tile) {
     uint32_t x, y;
@@ -725,8 +729,8 @@ __global__ void __launch_bounds__(kTraceBlock) k_trace_shadow(DagView g, const P
     if (own_lane(per_wave)) out[i] = dark;
 }
 
-// Rays of a wave: 64, or fewer while `count` rays make fewer than `waves`
-// waves.
+// Rays of a wave: 64, halved while that makes at most `waves` waves of `count`
+// rays.
 uint32_t rays_per_wave(uint64_t count, uint32_t waves) {
     uint32_t p = kWave;
     while (p > 1 && count * 2 <= (uint64_t)waves * p) p /= 2;
